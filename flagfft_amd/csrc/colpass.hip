@@ -25,11 +25,13 @@ __global__ __launch_bounds__(C * RB) __attribute__((amdgpu_waves_per_eu(WPE))) v
 
 namespace {
 
+constexpr int kColGroups = 256;  // one workgroup per CU
+
 struct ColEntry {
   int r, ra, rb, c, nch, wpe;
   bool dbl;
   const void *f;
-  int pref;  // default instance for first passes (1), later passes (2), both (3), neither (0)
+  int pref;  // default instance for first passes (1), later passes (2); 4: narrower tile for launches of few units
   int qvar;  // the persistent queue kernel's variant of this instance (k_queue in kernels.hip), -1 if none
   const void *fp;  // the instance with the DC / Nyquist pair modes, nullptr if none
 };
@@ -53,24 +55,43 @@ struct ColEntry {
 // passes (C-element stores) with 16; for R = 256 the first pass with 16
 // units (65-67 us per 2^24 pass against 72-73 with 64), later passes with 64
 // units in two exchange chunks (55-59 us against 62-65 with 16).
+//
+// A launch of fewer workgroups than CUs leaves the rest idle, and these
+// transforms (a few MB, in the caches) are bound by one workgroup's latency,
+// not by the row-segment width: the tile narrows until 256 workgroups are in
+// flight (entries with 4, in order of falling C).  1024 x 1024 C2C: 1024-point
+// columns in 32 workgroups of 32 units 21.3 us for the transform, 64 of 16
+// 16.5, 128 of 8 16.0, 256 of 4 15.5; 1024 x 4096: 31.5, 29.0, 29.4 (C = 8);
+// 65536 x 1: second pass of 64 / 32 / 16 units 14.2 / 11.2 / 10.5 us;
+// 2048 x 2048: 16 / 8 units 35.1 / 33.3.  Narrower 128-, 256- (first pass)
+// and 512-point FP32 tiles gave under 2 %.
 const ColEntry kColTable[] = {
     FLAGFFT_COLP(float, 8, 64, 64, 2, 2, 3),          // 4096: 64-byte runs, 135 KB LDS, 198 VGPRs
-    FLAGFFT_COL(float, 16, 32, 32, 2, 4, 2),          // 1024: 128-byte runs, 68 KB LDS, two workgroups per CU
+    FLAGFFT_COL(float, 16, 64, 32, 2, 2, 3),          // 2048: 128-byte runs, 135 KB LDS, 256 VGPRs
+    FLAGFFT_COL(float, 8, 64, 32, 2, 2, 4),           // 2048: 64-byte runs, 68 KB LDS
+    FLAGFFT_COL(float, 16, 32, 32, 2, 4, 6),          // 1024: 128-byte runs, 68 KB LDS, two workgroups per CU
     FLAGFFT_COL(float, 32, 32, 32, 2, 4, 1),          // 1024: 256-byte runs, 136 KB LDS, 1024 threads
     FLAGFFT_COL(float, 16, 32, 32, 1, 2, 0),          // 1024: 132 KB LDS, one workgroup per CU
-    FLAGFFT_COLQ(float, 8, 32, 32, 2, 4, 0, 0),       // 1024: 64-byte runs, 35 KB LDS, four workgroups per CU
+    FLAGFFT_COLQ(float, 8, 32, 32, 2, 4, 4, 0),       // 1024: 64-byte runs, 35 KB LDS, four workgroups per CU
     FLAGFFT_COL(float, 8, 32, 32, 1, 2, 0),           // 1024: 64-byte runs
-    FLAGFFT_COLQ(float, 16, 16, 16, 1, 2, 1, 2),      // 256: 128-byte runs, 33 KB LDS
+    FLAGFFT_COL(float, 4, 32, 32, 1, 2, 4),           // 1024: 32-byte runs, 128 threads
+    FLAGFFT_COLQ(float, 16, 16, 16, 1, 2, 5, 2),      // 256: 128-byte runs, 33 KB LDS
     FLAGFFT_COL(float, 32, 16, 16, 1, 4, 0),          // 256: 256-byte runs, 66 KB LDS
     FLAGFFT_COL(float, 64, 16, 16, 2, 4, 2),          // 256: 512-byte runs, 66 KB LDS, 1024 threads
     FLAGFFT_COLQ(float, 16, 32, 16, 1, 2, 3, 1),      // 512: 128-byte runs
     FLAGFFT_COLQ(float, 32, 16, 8, 1, 2, 3, 3),       // 128
     FLAGFFT_COL(float, 64, 8, 8, 1, 4, 3),            // 64: 512-byte runs
-    FLAGFFT_COLQ(float, 32, 8, 8, 1, 2, 0, 4),        // 64: 256-byte runs
+    FLAGFFT_COLQ(float, 32, 8, 8, 1, 2, 4, 4),        // 64: 256-byte runs
+    FLAGFFT_COL(float, 16, 8, 8, 1, 2, 4),            // 64: 128-byte runs
     FLAGFFT_COLQ(float, 64, 8, 4, 1, 2, 3, 5),        // 32: 512-byte runs
     FLAGFFT_COLQ(float, 64, 4, 4, 1, 2, 3, 6),        // 16: 512-byte runs
+    FLAGFFT_COL(double, 8, 32, 32, 2, 2, 3),          // 1024: 128-byte runs, 70 KB LDS, 219 VGPRs
+    FLAGFFT_COL(double, 4, 32, 32, 1, 2, 4),          // 1024: 64-byte runs
+    FLAGFFT_COL(double, 8, 32, 16, 1, 2, 3),          // 512: 128-byte runs
+    FLAGFFT_COL(double, 4, 32, 16, 1, 2, 4),          // 512: 64-byte runs
     FLAGFFT_COLQ(double, 16, 16, 16, 1, 2, 3, 7),     // 256: 256-byte runs, 66 KB LDS
-    FLAGFFT_COL(double, 8, 16, 16, 1, 2, 0),          // 256: 128-byte runs
+    FLAGFFT_COL(double, 8, 16, 16, 1, 2, 4),          // 256: 128-byte runs
+    FLAGFFT_COL(double, 4, 16, 16, 1, 2, 4),          // 256: 64-byte runs
     FLAGFFT_COL(double, 16, 16, 8, 1, 2, 3),          // 128
     FLAGFFT_COLQ(double, 32, 8, 8, 1, 2, 3, 9),       // 64
 };
@@ -94,22 +115,34 @@ int col_kernel_id(int64_t r, bool dbl, int units, bool first) {
 
 int col_kernel_id(int64_t r, bool dbl, int units) { return col_kernel_id(r, dbl, units, false); }
 
+int col_kernel_id_for(int64_t r, bool dbl, bool first, int64_t total_units) {
+  const int n = static_cast<int>(sizeof(kColTable) / sizeof(kColTable[0]));
+  int best = col_kernel_id(r, dbl, 0, first);
+  if (best < 0) return best;
+  for (int id = 0; id < n; ++id) {
+    const ColEntry &e = kColTable[id], &b = kColTable[best];
+    if (e.r != r || e.dbl != dbl || (e.pref & 4) == 0) continue;
+    if (total_units < static_cast<int64_t>(kColGroups) * b.c && e.c < b.c) best = id;
+  }
+  // 2048 points in 64 elements per thread are slower than the LDS
+  // super-stage's 16 once CUs run dry (2^21 x 1: 36 against 33 us, 2048 x 1024
+  // columns: 20 against 18); 4096 points are not (2^22 x 1: 40 against 44)
+  if (r == 2048 && total_units < static_cast<int64_t>(kColGroups) * kColTable[best].c) return -1;
+  return best;
+}
+
 int col_run_bytes(int64_t r, bool dbl, bool first) {
   const int id = col_kernel_id(r, dbl, 0, first);
   return id < 0 ? 0 : kColTable[id].c * (dbl ? 16 : 8);
 }
 
-int col_kernel_id_dividing(int64_t r, bool dbl, int64_t tcnt) {
-  const int n = static_cast<int>(sizeof(kColTable) / sizeof(kColTable[0]));
-  int any = -1;
-  for (int id = 0; id < n; ++id) {
-    const ColEntry &e = kColTable[id];
-    if (e.r != r || e.dbl != dbl || tcnt % e.c != 0) continue;
-    if (e.pref != 0) return id;
-    if (any < 0) any = id;
-  }
-  return any;
+bool col_tiles_divide(int64_t r, bool dbl, int64_t tcnt) {
+  for (const ColEntry &e : kColTable)
+    if (e.r == r && e.dbl == dbl && e.pref != 0 && tcnt % e.c == 0) return true;
+  return false;
 }
+
+int col_kernel_radix(int id) { return kColTable[id].r; }
 
 int col_queue_kernel_id(int64_t r, bool dbl) {
   const int n = static_cast<int>(sizeof(kColTable) / sizeof(kColTable[0]));

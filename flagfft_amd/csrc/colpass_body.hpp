@@ -63,6 +63,34 @@ __device__ __forceinline__ void pow8(V2<T> w, V2<T> *p) {
   p[7] = cmul(p[4], p[3]);
 }
 
+// Unit slot `sl` of tile `blk`: its position i in sequence bq + dq, where bq
+// is the sequence of the tile's first unit (uniform over the workgroup: the
+// addresses stay a uniform base plus 32-bit lane offsets; the host checks that
+// the sequences a tile touches span under 4 GiB).  A tile may run over the end
+// of a sequence into the next ones, so a sequence's units need not be a
+// multiple of C (129 half-spectrum columns of 256 slabs: 2064 whole tiles
+// where whole-sequence tiles were impossible and the LDS super-stage took
+// 38 us per 67 MB sweep); slots past the last unit repeat it and stay idle.
+struct ColUnit {
+  uint32_t bq, dq, i;
+  bool active;  // the slot has a unit
+  bool whole;   // every slot of the tile has one (uniform)
+};
+template <int C>
+__device__ __forceinline__ ColUnit col_unit(const StageArgs &a, int blk, int sl) {
+  const uint32_t u0 = static_cast<uint32_t>(blk) * C;
+  const uint32_t units = static_cast<uint32_t>(a.units);
+  const uint32_t u = min(u0 + static_cast<uint32_t>(sl), units - 1u);
+  ColUnit r;
+  r.bq = fdiv(u0, a.fd_tcnt);
+  const uint32_t b = fdiv(u, a.fd_tcnt);
+  r.dq = b - r.bq;
+  r.i = u - b * static_cast<uint32_t>(a.tcnt);
+  r.active = u0 + static_cast<uint32_t>(sl) < units;
+  r.whole = u0 + C <= units;
+  return r;
+}
+
 // Loads of tile `blk`: element e = t + RB j of the thread's unit (zero
 // outside the units and, for a Bluestein chirp source, past the user length).
 template <typename T, int C, int RA, int RB, bool PAIR = false>
@@ -70,12 +98,12 @@ __device__ __forceinline__ void col_load(const StageArgs &a, int blk, V2<T> (&x)
   const int tid = threadIdx.x;
   const int sl = tid % C;
   const int t = tid / C;
-  const int64_t u0 = static_cast<int64_t>(blk) * C;
-  const bool active = u0 + sl < a.units;
-  const uint32_t bq = fdiv(static_cast<uint32_t>(u0), a.fd_tcnt);
-  const uint32_t i = static_cast<uint32_t>(u0) - bq * static_cast<uint32_t>(a.tcnt) + sl;
+  const ColUnit un = col_unit<C>(a, blk, sl);
+  const uint32_t i = un.i;
   const uint32_t tcnt = static_cast<uint32_t>(a.tcnt);
-  const GlbC<T> *src = gc<T>(a.in) + static_cast<int64_t>(bq) * a.bs_in;
+  const uint32_t lead = un.dq * static_cast<uint32_t>(a.bs_in);
+  const uint32_t ia = i + lead;
+  const GlbC<T> *src = gc<T>(a.in) + static_cast<int64_t>(un.bq) * a.bs_in;
   const bool chirp_in = (a.src_mode & kSrcChirpFlag) != 0;
   const uint32_t nlog = static_cast<uint32_t>(a.nlog);
   if (PAIR && a.dc_nyq_pair == 2 && blk == 0 && sl == 0) {
@@ -96,10 +124,33 @@ __device__ __forceinline__ void col_load(const StageArgs &a, int blk, V2<T> (&x)
     }
     return;
   }
+  // (not the tile whose unit 0 is a pair: its lanes left above)
+  if (!chirp_in && un.whole && !(PAIR && a.dc_nyq_pair == 2 && blk == 0)) {
+#pragma unroll
+    for (int j = 0; j < RA; ++j) {
+      x[j] = ldt(src, ia + static_cast<uint32_t>(t + RB * j) * tcnt);
+      // 64 loads per thread, each of a row 64 rows further on (2 MB at a 32 KB
+      // pitch): the waves keep in step every 16 loads (issue order only, no
+      // wait for data), so a CU walks the pages together instead of each wave
+      // through its own.  4096-point columns of 4096^2 C2C 73 -> 63 us, the two
+      // passes of 2^24 104 + 73 -> 86 + 61 us.
+      if constexpr (RA >= 64) {
+        if (j % 16 == 15) {
+          __builtin_amdgcn_sched_barrier(0);
+          __builtin_amdgcn_s_barrier();
+          __builtin_amdgcn_sched_barrier(0);
+        }
+      }
+    }
+    return;
+  }
+  // elements from `lim` on are zero: all of an idle slot's, and those past the
+  // user length of a Bluestein chirp source
+  const uint32_t lim = !un.active ? 0u : chirp_in ? nlog + lead : ~0u;
 #pragma unroll
   for (int j = 0; j < RA; ++j) {
-    const uint32_t e = i + static_cast<uint32_t>(t + RB * j) * tcnt;
-    x[j] = (active && (!chirp_in || e < nlog)) ? ldt(src, e) : V2<T>{0, 0};
+    const uint32_t e = ia + static_cast<uint32_t>(t + RB * j) * tcnt;
+    x[j] = e < lim ? ldt(src, e) : V2<T>{0, 0};
   }
 }
 
@@ -121,13 +172,10 @@ __device__ __forceinline__ void col_rest(const StageArgs &a, int blk, V2<T> (&x)
   const int tid = threadIdx.x;
   const int sl = tid % C;
   const int t = tid / C;
-  // The host launches this kernel only when C divides tcnt (every tile lies
-  // in one sequence) and a sequence spans under 4 GiB: the sequence base is
-  // uniform and every element offset fits 32 bits.
   const int64_t u0 = static_cast<int64_t>(blk) * C;
-  const bool active = u0 + sl < a.units;
-  const uint32_t bq = fdiv(static_cast<uint32_t>(u0), a.fd_tcnt);
-  const uint32_t i = static_cast<uint32_t>(u0) - bq * static_cast<uint32_t>(a.tcnt) + sl;
+  const ColUnit un = col_unit<C>(a, blk, sl);
+  const bool active = un.active;
+  const uint32_t bq = un.bq, i = un.i;
   const bool first = a.p == a.ncol;
   const uint32_t k = i - fdiv(i, a.fd_p) * static_cast<uint32_t>(a.p);
   const uint32_t kt = first ? 0u : fdiv(k, a.fd_ncol);
@@ -369,6 +417,7 @@ __device__ __forceinline__ void col_rest(const StageArgs &a, int blk, V2<T> (&x)
     }
     if (active) {
       GlbC<T> *dst = gc<T>(a.out) + static_cast<int64_t>(bq) * a.bs_out;
+      const uint32_t lead = un.dq * static_cast<uint32_t>(a.bs_out);
       const uint32_t o0 = (i - k) * static_cast<uint32_t>(R) + k;
       const uint32_t pp = static_cast<uint32_t>(a.p);
       const GlbC<T> *bhat = gc<T>(a.bhat);
@@ -390,19 +439,34 @@ __device__ __forceinline__ void col_rest(const StageArgs &a, int blk, V2<T> (&x)
           }
         }
       } else {
+        // output index of y[m][q] within its sequence, less the lane's o0
+        auto rel = [&](int m, int q) __attribute__((always_inline)) {
+          return static_cast<uint32_t>(t + RB * m + RA * q) * pp;
+        };
+        if (a.dst_mode & kDstPointwiseFlag) {
 #pragma unroll
-        for (int m = 0; m < NM; ++m) {
-          const int k1 = t + RB * m;
+          for (int m = 0; m < NM; ++m) {
 #pragma unroll
-          for (int q = 0; q < RB; ++q) {
-            const uint32_t o = o0 + static_cast<uint32_t>(k1 + RA * q) * pp;
-            if (a.dst_mode & kDstPointwiseFlag) {
-              stt(dst, o, cconj(cmul(y[m][q], ldt(bhat, o))));
-            } else if (a.dst_mode & kDstChirpFlag) {
-              if (o < nlog) stt(dst, o, finish(cmul(cconj(y[m][q]), ldt(chirp, o))));
-            } else {
-              stt(dst, o, finish(y[m][q]));
+            for (int q = 0; q < RB; ++q) {
+              const uint32_t o = o0 + rel(m, q);
+              stt(dst, o + lead, cconj(cmul(y[m][q], ldt(bhat, o))));
             }
+          }
+        } else if (a.dst_mode & kDstChirpFlag) {
+#pragma unroll
+          for (int m = 0; m < NM; ++m) {
+#pragma unroll
+            for (int q = 0; q < RB; ++q) {
+              const uint32_t o = o0 + rel(m, q);
+              if (o < nlog) stt(dst, o + lead, finish(cmul(cconj(y[m][q]), ldt(chirp, o))));
+            }
+          }
+        } else {
+          const uint32_t oa = o0 + lead;
+#pragma unroll
+          for (int m = 0; m < NM; ++m) {
+#pragma unroll
+            for (int q = 0; q < RB; ++q) stt(dst, oa + rel(m, q), finish(y[m][q]));
           }
         }
       }

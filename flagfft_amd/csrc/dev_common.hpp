@@ -79,9 +79,11 @@ __device__ __forceinline__ LdsC<T> *lds_base() {
 __device__ __forceinline__ int lpad(int e) { return e + (e >> 5); }
 
 __device__ __forceinline__ int remap_block(int b, int nblocks, int enable) {
-  if (!enable || (nblocks & 7) != 0) return b;
-  // blocks are dispatched round-robin over the 8 XCDs: keep consecutive tiles on one XCD
-  return (b & 7) * (nblocks >> 3) + (b >> 3);
+  if (!enable) return b;
+  // blocks are dispatched round-robin over the 8 XCDs: keep consecutive tiles
+  // on one XCD (XCD x takes nblocks / 8 tiles, one more if x < nblocks mod 8)
+  const int x = b & 7;
+  return x * (nblocks >> 3) + min(x, nblocks & 7) + (b >> 3);
 }
 
 // Logical input element e: base source, then conjugation (inverse by the

@@ -121,6 +121,21 @@ size_t Step::pack_args(void *src, void *dst, unsigned char *buf, void *aux) cons
   return 0;
 }
 
+namespace {
+
+// Register-resident passes address a tile from the base of its first unit's
+// sequence with 32-bit offsets: the sequences a tile of `per` units touches
+// (more than one when `per` does not divide a sequence's units) must span
+// under 4 GiB.
+bool col_tiles_fit(int64_t tcnt, int64_t p, int R, int per, int64_t bs_in, int64_t bs_out, int64_t nseq, int eb) {
+  const int64_t reach = tcnt % per == 0 ? 0 : std::min((tcnt + per - 2) / tcnt, nseq - 1);
+  const int64_t bs = std::max(bs_in, bs_out);
+  if (reach > 0 && bs >= (int64_t{1} << 32)) return false;
+  return (reach * bs + std::max(tcnt, p) * R) * eb < (int64_t{1} << 32);
+}
+
+}  // namespace
+
 Step Step::rebatched(int64_t batch, int64_t built) const {
   Step s = *this;
   if (batch == built) return s;
@@ -136,9 +151,9 @@ Step Step::rebatched(int64_t batch, int64_t built) const {
       int per = 1, thr = 0, ebytes = 0;
       size_t lds = 0;
       col_kernel_shape(leaf_id, per, thr, lds, ebytes);
-      // a tile may end partially only when the pass has a single sequence
-      if (sa.tcnt % per != 0) throw std::logic_error("re-batched pass whose tiles would straddle sequences");
       s.sa.units = scale(sa.units);
+      if (!col_tiles_fit(sa.tcnt, sa.p, col_kernel_radix(leaf_id), per, sa.bs_in, sa.bs_out, s.sa.units / sa.tcnt, ebytes))
+        throw std::logic_error("re-batched pass whose tiles span 4 GiB");
       s.sa.nblocks = static_cast<int32_t>(blocks(s.sa.units, per));
       s.shape.grid = dim3(static_cast<unsigned>(s.sa.nblocks));
       break;
@@ -760,7 +775,9 @@ bool Builder::try_stage(const PassArgs &a, const std::vector<int> &radices, int 
                            (a.src_mode & 3) == kSrcComplex && (a.dst_mode & 3) == kDstComplex;
   int cid = !col_allowed        ? -1
             : opt_.queue_form ? col_queue_kernel_id(a.R, dbl())
-                              : col_kernel_id(a.R, dbl(), opt_.forced_units, a.p == 1);
+            : opt_.forced_units != 0
+                ? col_kernel_id(a.R, dbl(), opt_.forced_units, a.p == 1)
+                : col_kernel_id_for(a.R, dbl(), a.p == 1, a.units);
   // DC / Nyquist pair: one transform's single column pass over the n1 / 2
   // columns of the half spectrum (row pitch n1 / 2 + 1) but its Nyquist
   // column, which goes with column 0; the other side is a workspace of n1 / 2
@@ -790,17 +807,9 @@ bool Builder::try_stage(const PassArgs &a, const std::vector<int> &radices, int 
   int cunits = 0, cthreads = 0, cebytes = 0;
   size_t clds = 0;
   if (cid >= 0) col_kernel_shape(cid, cunits, cthreads, clds, cebytes);
-  // the default instance's tile does not divide the units of a sequence:
-  // another instance of the radix whose tile does
-  if (cid >= 0 && !pair && tcnt % cunits != 0 && a.units != tcnt && opt_.forced_units == 0 && !opt_.queue_form) {
-    cid = col_kernel_id_dividing(R, dbl(), tcnt);
-    if (cid >= 0) col_kernel_shape(cid, cunits, cthreads, clds, cebytes);
-  }
-  // the register-resident pass addresses a sequence from a uniform base with
-  // 32-bit offsets: its tiles may not straddle sequences, nor a sequence 4 GiB
   // (one sequence: the last tile may be partial, its lanes past the units idle)
-  const bool col_ok = cid >= 0 && (pair || tcnt % cunits == 0 || a.units == tcnt) &&
-                      std::max(tcnt, p) * R * eb() < (int64_t{1} << 32);
+  const bool col_ok =
+      cid >= 0 && col_tiles_fit(tcnt, p, R, cunits, a.gi.bs, a.go.bs, pair ? 1 : units / tcnt, eb());
   if (pair && !col_ok) throw std::logic_error("DC/Nyquist pair: the column pass does not fit");
   if (!col_ok && sid < 0) return false;
   if (col_ok) {

@@ -54,11 +54,15 @@ bool stage_kernel_fast(int id);
 // its units, threads, dynamic LDS bytes and element bytes; the kernel.
 int col_kernel_id(int64_t r, bool dbl, int units);
 int col_kernel_id(int64_t r, bool dbl, int units, bool first);
+// The default instance for a launch of total_units units: a narrower tile when
+// the default one would leave CUs without a workgroup, -1 where the LDS
+// super-stage is faster for so few.
+int col_kernel_id_for(int64_t r, bool dbl, bool first, int64_t total_units);
 // Row-segment bytes (units x element bytes) of the default instance, 0 if none.
 int col_run_bytes(int64_t r, bool dbl, bool first);
-// An instance of radix r whose units per workgroup divide tcnt (a default
-// instance first), or -1.
-int col_kernel_id_dividing(int64_t r, bool dbl, int64_t tcnt);
+// Whether the tile of some instance of radix r divides tcnt units.
+bool col_tiles_divide(int64_t r, bool dbl, int64_t tcnt);
+int col_kernel_radix(int id);
 void col_kernel_shape(int id, int &units, int &threads, size_t &lds_bytes, int &elem_bytes);
 const void *col_kernel(int id);
 // The same instance with the DC / Nyquist pair modes of a 2D real column pass

@@ -182,19 +182,23 @@ int column_segment_bytes(const std::vector<int> &rad, Prec p) {
 // row segments of 128 bytes or more, 3.0 to 4.2 with 64;
 // LDS super-stages at 2.2 to 3.5 by the row-segment bytes their tile reads;
 // the run-time-radix pass at about 1.1.
-// tcnt: units per sequence (n / r); a register-resident instance takes the
-// pass only when its units per workgroup divide it (one tile, one sequence).
+// tcnt: units per sequence (n / r).  A register-resident pass whose tiles do
+// not divide them runs all the same, its tiles crossing sequence ends, but is
+// not priced as one: 5- and 10-smooth lengths keep their chains of 25- to
+// 1000-point passes (250000 as [125, 125, 16] would take 28 us against 32 for
+// [100, 100, 25]).
 double pass_time(int64_t r, Prec p, bool first, const PlanOptions &o, int64_t tcnt) {
   std::vector<int> rad;
   if (o.generic_kernels) {
     // persistent-queue plans: register-resident queue instances, else the run-time-radix pass
     return (o.queue_form && col_queue_kernel_id(r, p == Prec::F64) >= 0) ? 1.0 / 4.0 : 1.0 / 1.1;
   }
-  if (o.stage_form != 2 && col_kernel_id(r, p == Prec::F64, 0) >= 0 &&
-      col_kernel_id_dividing(r, p == Prec::F64, tcnt) >= 0) {
+  if (o.stage_form != 2 && col_kernel_id(r, p == Prec::F64, 0) >= 0 && col_tiles_divide(r, p == Prec::F64, tcnt)) {
     // 64-byte segments (the 4096-point instance: 8 units of 32 KiB in one
-    // workgroup) run at 3.0 / 4.2
+    // workgroup) run at 3.0 / 4.2, the 2048-point FP32 instance (one workgroup
+    // per CU, as that one) at 3.1 / 4.1
     if (col_run_bytes(r, p == Prec::F64, first) < 128) return first ? 1.0 / 3.0 : 1.0 / 4.2;
+    if (r == 2048) return first ? 1.0 / 3.1 : 1.0 / 4.1;
     return first ? 1.0 / 3.8 : 1.0 / 4.6;
   }
   if (radix_factor(r, rad)) {
