@@ -4,6 +4,7 @@
 #include "kernels.hpp"
 
 #include <algorithm>
+#include <functional>
 #include <sstream>
 #include <stdexcept>
 
@@ -213,26 +214,41 @@ double pass_time(int64_t r, Prec p, bool first, const PlanOptions &o, int64_t tc
 // The split of n into 2-4 passes with the least total pass time; near ties
 // (2 %) go to fewer passes, then to the larger smallest factor.
 bool cheapest_split(int64_t n, Prec p, const PlanOptions &o, std::vector<int64_t> &best) {
-  const int64_t cap = pass_max(o, p);
+  // the super-radices that may take part, in falling order, each priced once
+  // as a first and as a later pass
+  struct Radix {
+    int64_t r;
+    double first, later;
+  };
+  std::vector<Radix> rs;
+  std::vector<int> tmp;
+  for (int64_t d = std::min(pass_max(o, p), n); d >= 2; --d)
+    if (n % d == 0 && radix_factor(d, tmp)) rs.push_back({d, pass_time(d, p, true, o, n / d), pass_time(d, p, false, o, n / d)});
   double best_t = 0.0;
   bool have = false;
-  for (int k = 2; k <= 4; ++k) {
-    std::vector<std::vector<int64_t>> all;
-    std::vector<int64_t> cur;
-    enum_splits(n, k, cap, cap, cur, all);
-    for (const auto &v : all) {
-      double tt = 0.0;
-      for (size_t i = 0; i < v.size(); ++i) tt += pass_time(v[i], p, i == 0, o, n / v[i]);
-      const bool better = !have || tt < best_t * 0.98 ||
-                          (tt <= best_t * 1.02 && v.size() == best.size() &&
-                           *std::min_element(v.begin(), v.end()) > *std::min_element(best.begin(), best.end()));
-      if (better) {
-        best = v;
-        best_t = tt;
-        have = true;
+  std::vector<int64_t> cur;
+  std::function<void(int64_t, int, size_t, double)> rec = [&](int64_t rest, int k, size_t from, double tt) {
+    for (size_t i = from; i < rs.size(); ++i) {
+      const Radix &x = rs[i];
+      if (rest % x.r != 0 || (k == 1 && x.r != rest)) continue;
+      const double t2 = tt + (cur.empty() ? x.first : x.later);
+      cur.push_back(x.r);
+      if (k > 1) {
+        rec(rest / x.r, k - 1, i, t2);
+      } else {
+        const bool better = !have || t2 < best_t * 0.98 ||
+                            (t2 <= best_t * 1.02 && cur.size() == best.size() &&
+                             *std::min_element(cur.begin(), cur.end()) > *std::min_element(best.begin(), best.end()));
+        if (better) {
+          best = cur;
+          best_t = t2;
+          have = true;
+        }
       }
+      cur.pop_back();
     }
-  }
+  };
+  for (int k = 2; k <= 4; ++k) rec(n, k, 0, 0.0);
   return have;
 }
 
