@@ -50,6 +50,12 @@ __device__ __forceinline__ void stt(GlbC<T> *base, uint32_t idx, V2<T> v) {
   stg(reinterpret_cast<GlbC<T> *>(b + idx * static_cast<uint32_t>(sizeof(V2<T>))), v);
 }
 
+template <typename T>
+__device__ __forceinline__ void stt_nt(GlbC<T> *base, uint32_t idx, V2<T> v) {
+  FLAGFFT_GLB char *b = reinterpret_cast<FLAGFFT_GLB char *>(base);
+  stg_nt<T>(reinterpret_cast<GlbC<T> *>(b + idx * static_cast<uint32_t>(sizeof(V2<T>))), v);
+}
+
 // p[j] = w^j for j < 8 (p[0] = 1), each at most three products deep.
 template <typename T>
 __device__ __forceinline__ void pow8(V2<T> w, V2<T> *p) {
@@ -126,22 +132,28 @@ __device__ __forceinline__ void col_load(const StageArgs &a, int blk, V2<T> (&x)
   }
   // (not the tile whose unit 0 is a pair: its lanes left above)
   if (!chirp_in && un.whole && !(PAIR && a.dc_nyq_pair == 2 && blk == 0)) {
+    auto load_tile = [&](auto ld) __attribute__((always_inline)) {
 #pragma unroll
-    for (int j = 0; j < RA; ++j) {
-      x[j] = ldt(src, ia + static_cast<uint32_t>(t + RB * j) * tcnt);
-      // 64 loads per thread, each of a row 64 rows further on (2 MB at a 32 KB
-      // pitch): the waves keep in step every 16 loads (issue order only, no
-      // wait for data), so a CU walks the pages together instead of each wave
-      // through its own.  4096-point columns of 4096^2 C2C 73 -> 63 us, the two
-      // passes of 2^24 104 + 73 -> 86 + 61 us.
-      if constexpr (RA >= 64) {
-        if (j % 16 == 15) {
-          __builtin_amdgcn_sched_barrier(0);
-          __builtin_amdgcn_s_barrier();
-          __builtin_amdgcn_sched_barrier(0);
+      for (int j = 0; j < RA; ++j) {
+        x[j] = ld(src, ia + static_cast<uint32_t>(t + RB * j) * tcnt);
+        // 64 loads per thread, each of a row 64 rows further on (2 MB at a 32 KB
+        // pitch): the waves keep in step every 16 loads (issue order only, no
+        // wait for data), so a CU walks the pages together instead of each wave
+        // through its own.  4096-point columns of 4096^2 C2C 73 -> 63 us, the two
+        // passes of 2^24 104 + 73 -> 86 + 61 us.
+        if constexpr (RA >= 64) {
+          if (j % 16 == 15) {
+            __builtin_amdgcn_sched_barrier(0);
+            __builtin_amdgcn_s_barrier();
+            __builtin_amdgcn_sched_barrier(0);
+          }
         }
       }
-    }
+    };
+    if (a.stream & kStreamIn)
+      load_tile([](const GlbC<T> *p, uint32_t e) __attribute__((always_inline)) { return ldt_nt<T>(p, e); });
+    else
+      load_tile([](const GlbC<T> *p, uint32_t e) __attribute__((always_inline)) { return ldt(p, e); });
     return;
   }
   // elements from `lim` on are zero: all of an idle slot's, and those past the
@@ -463,11 +475,17 @@ __device__ __forceinline__ void col_rest(const StageArgs &a, int blk, V2<T> (&x)
           }
         } else {
           const uint32_t oa = o0 + lead;
+          auto store_tile = [&](auto st) __attribute__((always_inline)) {
 #pragma unroll
-          for (int m = 0; m < NM; ++m) {
+            for (int m = 0; m < NM; ++m) {
 #pragma unroll
-            for (int q = 0; q < RB; ++q) stt(dst, oa + rel(m, q), finish(y[m][q]));
-          }
+              for (int q = 0; q < RB; ++q) st(dst, oa + rel(m, q), finish(y[m][q]));
+            }
+          };
+          if (a.stream & kStreamOut)
+            store_tile([](GlbC<T> *p, uint32_t e, V2<T> v) __attribute__((always_inline)) { stt_nt<T>(p, e, v); });
+          else
+            store_tile([](GlbC<T> *p, uint32_t e, V2<T> v) __attribute__((always_inline)) { stt(p, e, v); });
         }
       }
     }

@@ -44,6 +44,18 @@ __device__ __forceinline__ void stg(GlbC<T> *p, V2<T> v) {
   p->x = v.x;
   p->y = v.y;
 }
+// Non-temporal forms (see StreamHint).
+template <typename T>
+using Vec2 = T __attribute__((ext_vector_type(2)));
+template <typename T>
+__device__ __forceinline__ V2<T> ldg_nt(const GlbC<T> *p) {
+  const Vec2<T> v = __builtin_nontemporal_load(reinterpret_cast<const FLAGFFT_GLB Vec2<T> *>(p));
+  return V2<T>{v.x, v.y};
+}
+template <typename T>
+__device__ __forceinline__ void stg_nt(GlbC<T> *p, V2<T> v) {
+  __builtin_nontemporal_store(Vec2<T>{v.x, v.y}, reinterpret_cast<FLAGFFT_GLB Vec2<T> *>(p));
+}
 // Element `idx` of a table with a 32-bit index: the address stays a uniform
 // base plus one 32-bit lane offset (global_load with saddr), which keeps many
 // outstanding table loads cheap in registers.
@@ -51,6 +63,12 @@ template <typename T>
 __device__ __forceinline__ V2<T> ldt(const GlbC<T> *base, uint32_t idx) {
   const FLAGFFT_GLB char *b = reinterpret_cast<const FLAGFFT_GLB char *>(base);
   return ldg(reinterpret_cast<const GlbC<T> *>(b + idx * static_cast<uint32_t>(sizeof(V2<T>))));
+}
+
+template <typename T>
+__device__ __forceinline__ V2<T> ldt_nt(const GlbC<T> *base, uint32_t idx) {
+  const FLAGFFT_GLB char *b = reinterpret_cast<const FLAGFFT_GLB char *>(base);
+  return ldg_nt<T>(reinterpret_cast<const GlbC<T> *>(b + idx * static_cast<uint32_t>(sizeof(V2<T>))));
 }
 
 template <typename T>

@@ -9,8 +9,18 @@
 namespace flagfft {
 
 namespace {
-// Workgroups of the matrix-core kernel: each of its 4 waves loops over
-// transforms; 1024 groups keep every CU at its register-limited occupancy.
+// Inputs from half the Infinity Cache on are read with non-temporal loads: input
+// and workspace (or output) no longer fit it together.  4096^2 C2C 111 -> 103 us,
+// 256^3 C2C 143 -> 130, 2^24 C2C 143 -> 133; inputs of 64 MiB would lose (256^3
+// R2C 73 -> 79, 2048 x 4096 C2C 53.5 -> 56.5: the last pass over them often finds
+// them cached).
+constexpr int64_t kStreamInBytes = int64_t{128} << 20;
+// Outputs of single-pass rows up to this size are written with non-temporal
+// stores, which leave less to write back at the launch's end.  They do not stay in
+// the Infinity Cache, so that past it a transform that reads them next loses
+// more: forward and inverse in a row, 4096 x 256 13.2 -> 12.1 us, x 1024 28.9 ->
+// 23.9, x 1536 42.5 -> 41.7, x 2048 49.4 -> 53.4, x 4096 90.5 -> 94.
+constexpr int64_t kStreamOutBytes = int64_t{32} << 20;
 }  // namespace
 
 void hip_check(hipError_t e, const char *what) {
@@ -198,7 +208,59 @@ Step Step::rebatched(int64_t batch, int64_t built) const {
       s.shape = real_pre_shape(s.ra);
       break;
   }
+  s.input_bytes = scale(input_bytes);
+  s.output_bytes = scale(output_bytes);
+  s.set_stream_hints();
   return s;
+}
+
+void Step::set_stream_hints() {
+  bool in = input_bytes >= kStreamInBytes, out = output_bytes > 0;
+  auto bits = [&] { return (in ? kStreamIn : 0) | (out ? kStreamOut : 0); };
+  switch (kind) {
+    case Leaf: {
+      // as for Col below, whole lines: the last stage stores runs of tpu
+      // elements, N / radix apart (64 x 65536, 32-byte runs: 13.6 -> 30.3 us
+      // with the hint; 1000 x 16000, 800 bytes apart: 53.5 -> 56.4).  R2C rows
+      // (N + 1 bins) are never whole lines and gain all the same
+      const int64_t eb = dbl ? 16 : 8, tpu = shape.block.x / static_cast<unsigned>(la.C);
+      out = out && output_bytes <= kStreamOutBytes && tpu * eb >= 128 &&
+            (leaf_mode == kRowR2C || (la.odist * eb % 128 == 0 && leaf_kernel_last_stride(leaf_id) * eb % 128 == 0));
+      la.stream = bits();
+      break;
+    }
+    case RealPost:
+    case RealPre: ra.stream = bits(); break;
+    case Col: {
+      // whole 128-byte lines only: a tile's row segment under that, or across
+      // a line's end, meets the rest of the line from another workgroup, which
+      // a streamed line does not wait for (64-byte segments: second pass of
+      // 2^24 62 -> 86 us; 128 bytes: 2^20 x 16 107 -> 99 us, 512: 65536 x 256
+      // 93.5 -> 87.5).  Columns of 2D / 3D arrays keep plain stores: a
+      // following transform reads them sooner (256^3 there and back 249 -> 261)
+      int units = 0, threads = 0, eb = 0;
+      size_t lds = 0;
+      col_kernel_shape(leaf_id, units, threads, lds, eb);
+      in = in && static_cast<int64_t>(sa.tcnt) * eb % 128 == 0;
+      out = out && sa.ncol == 1 && units * eb % 128 == 0 && static_cast<int64_t>(sa.p) * eb % 128 == 0;
+      sa.stream = bits();
+      break;
+    }
+    default: break;
+  }
+}
+
+void Executable::mark_streams(int64_t in_bytes, int64_t out_bytes) {
+  int readers = 0;
+  for (const Step &s : steps) readers += s.src == kBufIn ? 1 : 0;
+  for (size_t i = 0; i < steps.size(); ++i) {
+    Step &s = steps[i];
+    s.input_bytes = s.src == kBufIn && readers == 1 ? in_bytes : 0;
+    s.output_bytes = s.dst == kBufOut ? out_bytes : 0;
+    for (size_t j = i + 1; j < steps.size(); ++j)
+      if (steps[j].src == kBufOut || steps[j].dst == kBufOut) s.output_bytes = 0;
+    s.set_stream_hints();
+  }
 }
 
 hipError_t Executable::run_batch(const void *in, void *out, void *const *wsp, int64_t batch, hipStream_t st) const {
@@ -1828,6 +1890,12 @@ std::unique_ptr<Executable> build_executable(const PlanTree &t, bool inverse, co
   }
   b.finish();
   ex->built_batch = t.desc.rank == 1 ? t.desc.batch : 1;
+  const int64_t last = t.desc.rank == 1 ? t.desc.n0 : t.desc.rank == 2 ? t.desc.n1 : t.desc.n2;
+  const int64_t lead = batch * (t.desc.rank == 1 ? 1 : t.desc.rank == 2 ? t.desc.n0 : t.desc.n0 * t.desc.n1);
+  const int64_t eb = elem_bytes(t.desc.prec);
+  const int64_t full = lead * last * eb, bins = lead * (last / 2 + 1) * eb;
+  ex->mark_streams(t.desc.real_fwd ? full / 2 : t.desc.real_inv ? bins : full,
+                   t.desc.real_fwd ? bins : t.desc.real_inv ? full / 2 : full);
   ex->resolve_kernels();
   if (allocate_ws) ex->allocate_workspaces();
   return ex;

@@ -77,6 +77,9 @@ struct Step {
   int64_t bytes_moved = 0;  // algorithmic HBM bytes of this launch (read + write)
   std::string label;
   const void *func = nullptr;  // kernel handle, set by Executable::resolve_kernels()
+  // bytes of the plan's input / output for the launch that alone reads the
+  // one / writes the other for good, else 0
+  int64_t input_bytes = 0, output_bytes = 0;
 
   static constexpr size_t kArgBytes = 1024;
   // The step's argument struct with its in/out (and aux) pointers set;
@@ -85,6 +88,8 @@ struct Step {
   // The same launch for `batch` sequences of a 1D plan built for `built` (every
   // per-batch count of a 1D plan is proportional to the batch).
   Step rebatched(int64_t batch, int64_t built) const;
+  // Set the launch's cache hints (StreamHint) from input_bytes and output_bytes.
+  void set_stream_hints();
 };
 
 class Executable {
@@ -104,6 +109,8 @@ class Executable {
   // Same launches as one hipGraph: recorded on first use, later calls patch
   // only the kernel nodes that read `in` or write `out`, then launch it.
   hipError_t run_graph(const void *in, void *out, hipStream_t st);
+  // Find the launches at the plan's ends and set their cache hints.
+  void mark_streams(int64_t in_bytes, int64_t out_bytes);
   // Look up every step's kernel handle and raise LDS limits (after building).
   void resolve_kernels();
   // 1D plans: run for `batch` sequences with caller-provided workspaces

@@ -44,6 +44,14 @@ enum DstMode : int32_t {
   kDstChirpFlag = 16,     // Bluestein end: e < n only, v = conj(v) * chirp[e] * scale, then base sink
 };
 
+// Cache hints (non-temporal loads / stores) of a launch at the plan's ends.
+//   out: the caller's output, written once and not read again by the plan.
+//        Plain stores leave it dirty in L2, where its write-backs meet the next
+//        launch's loads.
+//   in:  a large input, read once.  Plain loads leave it in the Infinity
+//        Cache, where it evicts the workspace that the next pass reads.
+enum StreamHint : int32_t { kStreamIn = 1, kStreamOut = 2 };
+
 struct Geometry {
   // element e of sequence (b, c) lives at base + b*bs + c*cs + e*es
   // (units of complex elements, or of reals for real sources / sinks)
@@ -132,6 +140,7 @@ struct LeafArgs {
   // in the imaginary part of bin 0 (R2C writes it there and leaves bin N
   // unwritten, C2R reads it there; both bins are real on that side)
   int32_t dc_nyq_pair;
+  int32_t stream;        // StreamHint bits
 };
 
 // Single-pass transform of length N = P L spread over P workgroups per
@@ -181,6 +190,7 @@ struct StageArgs {
   //   2: inverse: unit 0 reads Herm(A) + i Herm(B), Herm(V)_e = (V_e + conj V_-e) / 2,
   //      whose inverse transform is Re IFFT A + i Re IFFT B
   int32_t dc_nyq_pair;
+  int32_t stream;  // StreamHint bits (register-resident passes)
 };
 
 // Bluestein with the whole convolution in LDS (one sequence per workgroup).
@@ -244,6 +254,7 @@ struct RealPassArgs {
   const void *tw_lo, *tw_hi;
   int32_t tw_bits;
   int32_t conj_flag;
+  int32_t stream;       // StreamHint bits
 };
 
 // One job of the persistent mixed-length kernel: `nblocks` workgroup tiles of

@@ -783,8 +783,14 @@ __device__ __forceinline__ void real_post_body(const RealPassArgs &a, int blk, i
     const V2<T> ev{(zk.x + zc.x) * half, (zk.y + zc.y) * half};
     const V2<T> od = cmul_mi(V2<T>{(zk.x - zc.x) * half, (zk.y - zc.y) * half});
     const V2<T> wo = cmul(cmul(ldg(tw_hi + (k >> a.tw_bits)), ldg(tw_lo + (k & mask))), od);
-    stg(X + k * a.go.es, cadd(ev, wo));
-    if (2 * k != h) stg(X + (h - k) * a.go.es, cconj(csub(ev, wo)));
+    const V2<T> lo = cadd(ev, wo), hi = cconj(csub(ev, wo));
+    if (a.stream & kStreamOut) {
+      stg_nt<T>(X + k * a.go.es, lo);
+      if (2 * k != h) stg_nt<T>(X + (h - k) * a.go.es, hi);
+    } else {
+      stg(X + k * a.go.es, lo);
+      if (2 * k != h) stg(X + (h - k) * a.go.es, hi);
+    }
   }
 }
 
@@ -811,8 +817,9 @@ __device__ __forceinline__ void real_pre_body(const RealPassArgs &a, int blk, in
     const int64_t b = a.ncol == 1 ? q : q / a.ncol, c = q - b * a.ncol;
     const GlbC<T> *Xs = gc<T>(a.in) + b * a.gi.bs + c * a.gi.cs;
     GlbC<T> *Zo = gc<T>(a.out) + b * a.go.bs + c * a.go.cs;
-    V2<T> xk = ldg(Xs + k * a.gi.es);
-    V2<T> xh = ldg(Xs + (h - k) * a.gi.es);
+    const GlbC<T> *pk = Xs + k * a.gi.es, *ph = Xs + (h - k) * a.gi.es;
+    V2<T> xk = (a.stream & kStreamIn) ? ldg_nt<T>(pk) : ldg(pk);
+    V2<T> xh = (a.stream & kStreamIn) ? ldg_nt<T>(ph) : ldg(ph);
     if (k == 0) {
       xk.y = T(0);
       xh.y = T(0);

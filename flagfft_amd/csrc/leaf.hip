@@ -49,6 +49,7 @@ __global__ __launch_bounds__(kMaxBlockThreads) void k_leaf(const LeafArgs a) {
   const T scale = static_cast<T>(a.scale);
   const GlbC<T> *wn = gc<T>(a.aux);
   const GlbC<T> *tw = gc<T>(a.tw);
+  V2<T> twr[RS::template pow_total<E>()];  // base twiddles of the inner stages
   // split-spectrum passes: thread t handles k = t + i TPU, k <= N/2; every
   // table (and, for C2R, input) load of them is issued before any is used,
   // so their latencies overlap instead of one round trip per k
@@ -64,14 +65,21 @@ __global__ __launch_bounds__(kMaxBlockThreads) void k_leaf(const LeafArgs a) {
   if constexpr (Mode == kLeafC2R) {
     // fused pre-process into LDS (conjugated: the inverse runs as a forward transform)
     V2<T> xks[NK], xhs[NK];
+    auto load_bins = [&](auto ld) __attribute__((always_inline)) {
 #pragma unroll
-    for (int i = 0; i < NK; ++i) {
-      const int k = t + i * TPU;
-      const bool ok = active && k <= N / 2;
-      xks[i] = ok ? ldg(src + k) : V2<T>{0, 0};
-      // a paired row carries X_N's real part in the imaginary part of X_0
-      xhs[i] = (ok && !(k == 0 && a.dc_nyq_pair)) ? ldg(src + (N - k)) : V2<T>{0, 0};
-    }
+      for (int i = 0; i < NK; ++i) {
+        // (lanes past N / 2 read its bin; idle slots point at sequence 0.  A
+        // paired row carries X_N's real part in Im X_0: bin 0 stands for bin N)
+        const int k = min(t + i * TPU, N / 2);
+        xks[i] = ld(src + k);
+        xhs[i] = ld(src + (k == 0 && a.dc_nyq_pair ? 0 : N - k));
+      }
+    };
+    if (a.stream & kStreamIn)
+      load_bins([](const GlbC<T> *p) __attribute__((always_inline)) { return ldg_nt<T>(p); });
+    else
+      load_bins([](const GlbC<T> *p) __attribute__((always_inline)) { return ldg(p); });
+    prefetch_base_twiddles<T, E, TPU, RS>(twr, tw, t);
 #pragma unroll
     for (int i = 0; i < NK; ++i) {
       const int k = t + i * TPU;
@@ -105,27 +113,40 @@ __global__ __launch_bounds__(kMaxBlockThreads) void k_leaf(const LeafArgs a) {
     constexpr int NB = N / RR;
     constexpr int MB = RS::template butterflies<E>(s);
     V2<T> x[MB * RR];
+    if constexpr (s == 0 && Mode != kLeafC2R) {
+      auto load_row = [&](auto ld) __attribute__((always_inline)) {
+#pragma unroll
+        for (int m = 0; m < MB; ++m) {
+          // every lane loads, without a branch: those past the last butterfly
+          // repeat it, idle slots point at sequence 0
+          const int b = (m + 1) * TPU <= NB ? t + m * TPU : min(t + m * TPU, NB - 1);
+#pragma unroll
+          for (int j = 0; j < RR; ++j) x[m * RR + j] = ld(src + (b + j * NB));
+        }
+      };
+      if (a.stream & kStreamIn)
+        load_row([](const GlbC<T> *p) __attribute__((always_inline)) { return ldg_nt<T>(p); });
+      else
+        load_row([](const GlbC<T> *p) __attribute__((always_inline)) { return ldg(p); });
+      prefetch_base_twiddles<T, E, TPU, RS>(twr, tw, t);
+    }
 #pragma unroll
     for (int m = 0; m < MB; ++m) {
       const int b = t + m * TPU;
       if (b < NB) {
+        if constexpr (s > 0 || Mode == kLeafC2R) {
 #pragma unroll
-        for (int j = 0; j < RR; ++j) {
-          const int e = b + j * NB;
-          V2<T> v;
-          if constexpr (s == 0 && Mode != kLeafC2R) {
-            v = active ? ldg(src + e) : V2<T>{0, 0};
-            if (a.conj_in) v.y = -v.y;
-          } else {
-            v = ldc(buf + lpad(e));
-          }
-          x[m * RR + j] = v;
+          for (int j = 0; j < RR; ++j) x[m * RR + j] = ldc(buf + lpad(b + j * NB));
+        } else if (a.conj_in) {
+#pragma unroll
+          for (int j = 0; j < RR; ++j) x[m * RR + j].y = -x[m * RR + j].y;
         }
         if constexpr (q > 1) {
           // w^(j k) by binary powers of the butterfly's base twiddle: one
-          // table load per butterfly instead of RR - 1
-          constexpr int ts = N / (q * RR);
-          twiddle_powers<T, RR>(&x[m * RR], ldg(tw + (b % q) * ts));
+          // table load per butterfly instead of RR - 1, in flight with the data
+          // since the start (a load in each stage is a table round trip after
+          // each barrier)
+          twiddle_powers<T, RR>(&x[m * RR], twr[RS::template pow_offset<E>(s) + m]);
         }
         dft<RR>(&x[m * RR]);
       }
@@ -173,6 +194,9 @@ __global__ __launch_bounds__(kMaxBlockThreads) void k_leaf(const LeafArgs a) {
         }
         if (k == 0 && a.dc_nyq_pair) {
           stg(dst, V2<T>{lo.x, hi.x});  // X_0 and X_N are real: one slot
+        } else if (a.stream & kStreamOut) {
+          stg_nt<T>(dst + k, lo);
+          if (2 * k != N) stg_nt<T>(dst + (N - k), hi);
         } else {
           stg(dst + k, lo);
           if (2 * k != N) stg(dst + (N - k), hi);
@@ -180,22 +204,28 @@ __global__ __launch_bounds__(kMaxBlockThreads) void k_leaf(const LeafArgs a) {
       }
     } else if (active) {
       // last stage: q * RR == N, so k == b and the output index is b + j q
+      auto store_row = [&](auto st) __attribute__((always_inline)) {
 #pragma unroll
-      for (int m = 0; m < MB; ++m) {
-        const int b = t + m * TPU;
-        if (b < NB) {
+        for (int m = 0; m < MB; ++m) {
+          const int b = t + m * TPU;
+          if (b < NB) {
 #pragma unroll
-          for (int j = 0; j < RR; ++j) {
-            V2<T> v = x[m * RR + j];
-            if (a.conj_out) v.y = -v.y;
-            if (scale != T(1)) {
-              v.x *= scale;
-              v.y *= scale;
+            for (int j = 0; j < RR; ++j) {
+              V2<T> v = x[m * RR + j];
+              if (a.conj_out) v.y = -v.y;
+              if (scale != T(1)) {
+                v.x *= scale;
+                v.y *= scale;
+              }
+              st(dst + b + j * q, v);
             }
-            stg(dst + b + j * q, v);
           }
         }
-      }
+      };
+      if (a.stream & kStreamOut)
+        store_row([](GlbC<T> *p, V2<T> v) __attribute__((always_inline)) { stg_nt<T>(p, v); });
+      else
+        store_row([](GlbC<T> *p, V2<T> v) __attribute__((always_inline)) { stg(p, v); });
     }
   });
 }
@@ -299,6 +329,13 @@ int leaf_kernel_id(const std::vector<int> &radices) {
 }
 
 int leaf_kernel_ept(int id, bool dbl) { return dbl ? kLeafTable[id].e64 : kLeafTable[id].e32; }
+
+int leaf_kernel_last_stride(int id) {
+  const LeafEntry &e = kLeafTable[id];
+  int q = 1;
+  for (int j = 0; j + 1 < e.nrad; ++j) q *= e.rad[j];
+  return q;
+}
 
 const void *leaf_kernel(bool dbl, int id, int mode) { return kLeafTable[id].f[dbl ? 1 : 0][mode]; }
 
