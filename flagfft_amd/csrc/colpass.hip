@@ -14,11 +14,15 @@ namespace dev {
 
 // WPE: waves per SIMD the register allocation must leave room for (two
 // workgroups of C * RB threads per CU: C * RB / 128).
-// PAIR: the instance with the DC / Nyquist pair modes of a 2D real column
-// pass (a separate instance keeps that code out of every other pass).
-template <typename T, int C, int RA, int RB, int NCH, int WPE, int TWM, bool PAIR>
+template <typename T, int C, int RA, int RB, int NCH, int WPE, int MODE>
 __global__ __launch_bounds__(C * RB) __attribute__((amdgpu_waves_per_eu(WPE))) void k_col(const StageArgs a) {
-  col_body<T, C, RA, RB, NCH, TWM, PAIR>(a, remap_block(blockIdx.x, a.nblocks, a.xcd_remap));
+  col_body<T, C, RA, RB, NCH, MODE>(a, remap_block(blockIdx.x, a.nblocks, a.xcd_remap));
+}
+
+// The convolution launch of a two-pass Bluestein chain (square instances).
+template <typename T, int C, int RA, int NCH, int WPE>
+__global__ __launch_bounds__(C * RA) __attribute__((amdgpu_waves_per_eu(WPE))) void k_col_conv(const StageArgs a) {
+  col_conv_body<T, C, RA, NCH>(a, remap_block(blockIdx.x, a.nblocks, a.xcd_remap));
 }
 
 }  // namespace dev
@@ -30,21 +34,32 @@ constexpr int kColGroups = 256;  // one workgroup per CU
 struct ColEntry {
   int r, ra, rb, c, nch, wpe;
   bool dbl;
-  const void *f;
+  const void *f;   // plain passes
+  const void *fb;  // ends of Bluestein chains
   int pref;  // default instance for first passes (1), later passes (2); 4: narrower tile for launches of few units
   int qvar;  // the persistent queue kernel's variant of this instance (k_queue in kernels.hip), -1 if none
   const void *fp;  // the instance with the DC / Nyquist pair modes, nullptr if none
+  const void *fc;  // the convolution launch of a Bluestein chain (square instances), nullptr if none
 };
 
-#define FLAGFFT_COL(T, C, RA, RB, NCH, WPE, PREF)                                                                  \
-  {RA * RB, RA, RB, C, NCH, WPE, sizeof(T) == 8, (const void *)dev::k_col<T, C, RA, RB, NCH, WPE, 1, false>, PREF, \
-   -1, nullptr}
-#define FLAGFFT_COLP(T, C, RA, RB, NCH, WPE, PREF)                                                                 \
-  {RA * RB, RA, RB, C, NCH, WPE, sizeof(T) == 8, (const void *)dev::k_col<T, C, RA, RB, NCH, WPE, 1, false>, PREF, \
-   -1, (const void *)dev::k_col<T, C, RA, RB, NCH, WPE, 1, true>}
-#define FLAGFFT_COLQ(T, C, RA, RB, NCH, WPE, PREF, QVAR)                                                           \
-  {RA * RB, RA, RB, C, NCH, WPE, sizeof(T) == 8, (const void *)dev::k_col<T, C, RA, RB, NCH, WPE, 1, false>, PREF, \
-   QVAR, nullptr}
+#define FLAGFFT_COL(T, C, RA, RB, NCH, WPE, PREF) \
+  {RA * RB, RA, RB, C, NCH, WPE, sizeof(T) == 8, (const void *)dev::k_col<T, C, RA, RB, NCH, WPE, dev::kColPlain>, \
+   (const void *)dev::k_col<T, C, RA, RB, NCH, WPE, dev::kColBluestein>, PREF, \
+   -1, nullptr, nullptr}
+#define FLAGFFT_COLP(T, C, RA, RB, NCH, WPE, PREF) \
+  {RA * RB, RA, RB, C, NCH, WPE, sizeof(T) == 8, (const void *)dev::k_col<T, C, RA, RB, NCH, WPE, dev::kColPlain>, \
+   (const void *)dev::k_col<T, C, RA, RB, NCH, WPE, dev::kColBluestein>, PREF, \
+   -1, (const void *)dev::k_col<T, C, RA, RB, NCH, WPE, dev::kColPair>, \
+   (const void *)dev::k_col_conv<T, C, RA, NCH, WPE>}
+#define FLAGFFT_COLQ(T, C, RA, RB, NCH, WPE, PREF, QVAR) \
+  {RA * RB, RA, RB, C, NCH, WPE, sizeof(T) == 8, (const void *)dev::k_col<T, C, RA, RB, NCH, WPE, dev::kColPlain>, \
+   (const void *)dev::k_col<T, C, RA, RB, NCH, WPE, dev::kColBluestein>, PREF, \
+   QVAR, nullptr, nullptr}
+
+#define FLAGFFT_COLC(T, C, RA, NCH, WPE, PREF, QVAR) \
+  {RA * RA, RA, RA, C, NCH, WPE, sizeof(T) == 8, (const void *)dev::k_col<T, C, RA, RA, NCH, WPE, dev::kColPlain>, \
+   (const void *)dev::k_col<T, C, RA, RA, NCH, WPE, dev::kColBluestein>, PREF, \
+   QVAR, nullptr, (const void *)dev::k_col_conv<T, C, RA, NCH, WPE>}
 
 // Measured on MI355X (2^20 x 16 and 2^24 C2C FP32): for R = 4096 (64 x 64
 // in registers, 198 VGPRs, one 512-thread workgroup per CU) 8 units per
@@ -69,31 +84,31 @@ const ColEntry kColTable[] = {
     FLAGFFT_COLP(float, 8, 64, 64, 2, 2, 3),          // 4096: 64-byte runs, 135 KB LDS, 198 VGPRs
     FLAGFFT_COL(float, 16, 64, 32, 2, 2, 3),          // 2048: 128-byte runs, 135 KB LDS, 256 VGPRs
     FLAGFFT_COL(float, 8, 64, 32, 2, 2, 4),           // 2048: 64-byte runs, 68 KB LDS
-    FLAGFFT_COL(float, 16, 32, 32, 2, 4, 6),          // 1024: 128-byte runs, 68 KB LDS, two workgroups per CU
+    FLAGFFT_COLC(float, 16, 32, 2, 4, 6, -1),          // 1024: 128-byte runs, 68 KB LDS, two workgroups per CU
     FLAGFFT_COL(float, 32, 32, 32, 2, 4, 1),          // 1024: 256-byte runs, 136 KB LDS, 1024 threads
     FLAGFFT_COL(float, 16, 32, 32, 1, 2, 0),          // 1024: 132 KB LDS, one workgroup per CU
-    FLAGFFT_COLQ(float, 8, 32, 32, 2, 4, 4, 0),       // 1024: 64-byte runs, 35 KB LDS, four workgroups per CU
+    FLAGFFT_COLC(float, 8, 32, 2, 4, 4, 0),       // 1024: 64-byte runs, 35 KB LDS, four workgroups per CU
     FLAGFFT_COL(float, 8, 32, 32, 1, 2, 0),           // 1024: 64-byte runs
-    FLAGFFT_COL(float, 4, 32, 32, 1, 2, 4),           // 1024: 32-byte runs, 128 threads
-    FLAGFFT_COLQ(float, 16, 16, 16, 1, 2, 5, 2),      // 256: 128-byte runs, 33 KB LDS
+    FLAGFFT_COLC(float, 4, 32, 1, 2, 4, -1),           // 1024: 32-byte runs, 128 threads
+    FLAGFFT_COLC(float, 16, 16, 1, 2, 5, 2),      // 256: 128-byte runs, 33 KB LDS
     FLAGFFT_COL(float, 32, 16, 16, 1, 4, 0),          // 256: 256-byte runs, 66 KB LDS
     FLAGFFT_COL(float, 64, 16, 16, 2, 4, 2),          // 256: 512-byte runs, 66 KB LDS, 1024 threads
     FLAGFFT_COLQ(float, 16, 32, 16, 1, 2, 3, 1),      // 512: 128-byte runs
     FLAGFFT_COLQ(float, 32, 16, 8, 1, 2, 3, 3),       // 128
     FLAGFFT_COL(float, 64, 8, 8, 1, 4, 3),            // 64: 512-byte runs
-    FLAGFFT_COLQ(float, 32, 8, 8, 1, 2, 4, 4),        // 64: 256-byte runs
+    FLAGFFT_COLC(float, 32, 8, 1, 2, 4, 4),        // 64: 256-byte runs
     FLAGFFT_COL(float, 16, 8, 8, 1, 2, 4),            // 64: 128-byte runs
     FLAGFFT_COLQ(float, 64, 8, 4, 1, 2, 3, 5),        // 32: 512-byte runs
     FLAGFFT_COLQ(float, 64, 4, 4, 1, 2, 3, 6),        // 16: 512-byte runs
-    FLAGFFT_COL(double, 8, 32, 32, 2, 2, 3),          // 1024: 128-byte runs, 70 KB LDS, 219 VGPRs
+    FLAGFFT_COLC(double, 8, 32, 2, 2, 3, -1),          // 1024: 128-byte runs, 70 KB LDS, 219 VGPRs
     FLAGFFT_COL(double, 4, 32, 32, 1, 2, 4),          // 1024: 64-byte runs
     FLAGFFT_COL(double, 8, 32, 16, 1, 2, 3),          // 512: 128-byte runs
     FLAGFFT_COL(double, 4, 32, 16, 1, 2, 4),          // 512: 64-byte runs
-    FLAGFFT_COLQ(double, 16, 16, 16, 1, 2, 3, 7),     // 256: 256-byte runs, 66 KB LDS
-    FLAGFFT_COL(double, 8, 16, 16, 1, 2, 4),          // 256: 128-byte runs
-    FLAGFFT_COL(double, 4, 16, 16, 1, 2, 4),          // 256: 64-byte runs
+    FLAGFFT_COLC(double, 16, 16, 1, 2, 3, 7),     // 256: 256-byte runs, 66 KB LDS
+    FLAGFFT_COLC(double, 8, 16, 1, 2, 4, -1),          // 256: 128-byte runs
+    FLAGFFT_COLC(double, 4, 16, 1, 2, 4, -1),          // 256: 64-byte runs
     FLAGFFT_COL(double, 16, 16, 8, 1, 2, 3),          // 128
-    FLAGFFT_COLQ(double, 32, 8, 8, 1, 2, 3, 9),       // 64
+    FLAGFFT_COLC(double, 32, 8, 1, 2, 3, 9),       // 64
 };
 
 }  // namespace
@@ -115,8 +130,12 @@ int col_kernel_id(int64_t r, bool dbl, int units, bool first) {
 
 int col_kernel_id(int64_t r, bool dbl, int units) { return col_kernel_id(r, dbl, units, false); }
 
-int col_kernel_id_for(int64_t r, bool dbl, bool first, int64_t total_units) {
+int col_kernel_id_for(int64_t r, bool dbl, bool first, int64_t total_units, bool rows) {
   const int n = static_cast<int>(sizeof(kColTable) / sizeof(kColTable[0]));
+  // first 256-point passes of long 1D batches read 512-byte runs as the later
+  // ones do (65536 x 128 48.0 -> 45.3 us, x 256 95.5 -> 89.4, x 64 the same; 256^3
+  // columns lose 3 %)
+  if (rows && first && r == 256 && !dbl && total_units >= 32768) first = false;
   int best = col_kernel_id(r, dbl, 0, first);
   if (best < 0) return best;
   for (int id = 0; id < n; ++id) {
@@ -140,6 +159,13 @@ bool col_tiles_divide(int64_t r, bool dbl, int64_t tcnt) {
   for (const ColEntry &e : kColTable)
     if (e.r == r && e.dbl == dbl && e.pref != 0 && tcnt % e.c == 0) return true;
   return false;
+}
+
+std::vector<int64_t> col_kernel_radices(bool dbl) {
+  std::vector<int64_t> v;
+  for (const ColEntry &e : kColTable)
+    if (e.dbl == dbl) v.push_back(e.r);
+  return v;
 }
 
 int col_kernel_radix(int id) { return kColTable[id].r; }
@@ -170,7 +196,20 @@ void col_kernel_shape(int id, int &units, int &threads, size_t &lds_bytes, int &
   lds_bytes = static_cast<size_t>(need) * static_cast<size_t>(elem_bytes);
 }
 
-const void *col_kernel(int id) { return kColTable[id].f; }
+const void *col_conv_kernel(int id) { return kColTable[id].fc; }
+
+int col_conv_kernel_id(int64_t r, bool dbl, int64_t total_units) {
+  const int n = static_cast<int>(sizeof(kColTable) / sizeof(kColTable[0]));
+  int best = -1;
+  for (int id = 0; id < n; ++id) {
+    const ColEntry &e = kColTable[id];
+    if (e.r != r || e.dbl != dbl || e.fc == nullptr) continue;
+    if (best < 0 || (total_units < static_cast<int64_t>(kColGroups) * kColTable[best].c && e.c < kColTable[best].c)) best = id;
+  }
+  return best;
+}
+
+const void *col_kernel(int id, bool bluestein) { return bluestein ? kColTable[id].fb : kColTable[id].f; }
 
 const void *col_pair_kernel(int id) { return kColTable[id].fp; }
 
@@ -179,10 +218,15 @@ int col_pair_kernel_id(int64_t r, bool dbl) {
   return id >= 0 && kColTable[id].fp != nullptr ? id : -1;
 }
 
-std::string col_kernel_targs(int id, bool pair) {
+std::string col_conv_targs(int id) {
+  const ColEntry &e = kColTable[id];
+  return std::to_string(e.c) + "," + std::to_string(e.ra) + "," + std::to_string(e.nch) + "," + std::to_string(e.wpe);
+}
+
+std::string col_kernel_targs(int id, int mode) {
   const ColEntry &e = kColTable[id];
   return std::to_string(e.c) + "," + std::to_string(e.ra) + "," + std::to_string(e.rb) + "," + std::to_string(e.nch) +
-         "," + std::to_string(e.wpe) + ",1," + (pair ? "true" : "false");
+         "," + std::to_string(e.wpe) + "," + std::to_string(mode);
 }
 
 }  // namespace flagfft

@@ -56,18 +56,32 @@ __device__ __forceinline__ void stt_nt(GlbC<T> *base, uint32_t idx, V2<T> v) {
   stg_nt<T>(reinterpret_cast<GlbC<T> *>(b + idx * static_cast<uint32_t>(sizeof(V2<T>))), v);
 }
 
-// p[j] = w^j for j < 8 (p[0] = 1), each at most three products deep.
-template <typename T>
-__device__ __forceinline__ void pow8(V2<T> w, V2<T> *p) {
+// p[j] = w^j for j < N <= 8 (p[0] = 1), at most two products from w, w^2 and w^4,
+// which get(b) gives (b = 0, 1, 2; EXACT), or from w alone.  Powers of one
+// rounded w carry its error up to j times over: FP32 chains of 2^20 points have
+// a relative L2 error of 2.75e-7 that way and 2.03e-7 with the three values,
+// for 1 % of their time.  Passes of 16 elements per thread keep the one load
+// (with three, twice the loads of their data: second pass of 65536 x 256 44.5 ->
+// 46.7 us) unless they stand in for the run-time-radix pass with its table of
+// all powers, in Bluestein chains of real sequences.
+template <int N, bool EXACT, typename T, typename Get>
+__device__ __forceinline__ void powers(Get get, V2<T> *p) {
   p[0] = V2<T>{1, 0};
-  p[1] = w;
-  p[2] = cmul(w, w);
-  p[3] = cmul(p[2], w);
-  p[4] = cmul(p[2], p[2]);
-  p[5] = cmul(p[4], w);
-  p[6] = cmul(p[3], p[3]);
-  p[7] = cmul(p[4], p[3]);
+  if constexpr (N > 1) p[1] = get(0);
+  if constexpr (N > 2) p[2] = EXACT ? get(1) : cmul(p[1], p[1]);
+  if constexpr (N > 3) p[3] = cmul(p[2], p[1]);
+  if constexpr (N > 4) p[4] = EXACT ? get(2) : cmul(p[2], p[2]);
+  if constexpr (N > 5) p[5] = cmul(p[4], p[1]);
+  if constexpr (N > 6) p[6] = EXACT ? cmul(p[4], p[2]) : cmul(p[3], p[3]);
+  if constexpr (N > 7) p[7] = cmul(p[4], p[3]);
 }
+
+// What an instance runs besides plain passes: the DC / Nyquist pair of a 2D real
+// column pass (StageArgs::dc_nyq_pair), or the ends of Bluestein chains (chirp
+// source, pointwise and chirp sinks).  Instances of their own: the sinks' table
+// values cost the 64 x 256-point pass its second workgroup per CU (42 -> 54 us of
+// 65536 x 256).
+enum ColMode : int { kColPlain = 0, kColPair = 1, kColBluestein = 2 };
 
 // Unit slot `sl` of tile `blk`: its position i in sequence bq + dq, where bq
 // is the sequence of the tile's first unit (uniform over the workgroup: the
@@ -98,8 +112,8 @@ __device__ __forceinline__ ColUnit col_unit(const StageArgs &a, int blk, int sl)
 }
 
 // Loads of tile `blk`: element e = t + RB j of the thread's unit (zero
-// outside the units and, for a Bluestein chirp source, past the user length).
-template <typename T, int C, int RA, int RB, bool PAIR = false>
+// outside the units); a Bluestein chirp source comes with its chirp.
+template <typename T, int C, int RA, int RB, int MODE>
 __device__ __forceinline__ void col_load(const StageArgs &a, int blk, V2<T> (&x)[RA]) {
   const int tid = threadIdx.x;
   const int sl = tid % C;
@@ -110,9 +124,9 @@ __device__ __forceinline__ void col_load(const StageArgs &a, int blk, V2<T> (&x)
   const uint32_t lead = un.dq * static_cast<uint32_t>(a.bs_in);
   const uint32_t ia = i + lead;
   const GlbC<T> *src = gc<T>(a.in) + static_cast<int64_t>(un.bq) * a.bs_in;
-  const bool chirp_in = (a.src_mode & kSrcChirpFlag) != 0;
+  const bool chirp_in = MODE == kColBluestein && (a.src_mode & kSrcChirpFlag) != 0;
   const uint32_t nlog = static_cast<uint32_t>(a.nlog);
-  if (PAIR && a.dc_nyq_pair == 2 && blk == 0 && sl == 0) {
+  if (MODE == kColPair && a.dc_nyq_pair == 2 && blk == 0 && sl == 0) {
     // unit 0 of an inverse 2D real column pass: Herm(A) + i Herm(B) for the
     // DC column A (column 0) and the Nyquist column B (column `units`)
     constexpr int R = RA * RB;
@@ -131,7 +145,7 @@ __device__ __forceinline__ void col_load(const StageArgs &a, int blk, V2<T> (&x)
     return;
   }
   // (not the tile whose unit 0 is a pair: its lanes left above)
-  if (!chirp_in && un.whole && !(PAIR && a.dc_nyq_pair == 2 && blk == 0)) {
+  if (!chirp_in && un.whole && !(MODE == kColPair && a.dc_nyq_pair == 2 && blk == 0)) {
     auto load_tile = [&](auto ld) __attribute__((always_inline)) {
 #pragma unroll
       for (int j = 0; j < RA; ++j) {
@@ -156,119 +170,112 @@ __device__ __forceinline__ void col_load(const StageArgs &a, int blk, V2<T> (&x)
       load_tile([](const GlbC<T> *p, uint32_t e) __attribute__((always_inline)) { return ldt(p, e); });
     return;
   }
-  // elements from `lim` on are zero: all of an idle slot's, and those past the
-  // user length of a Bluestein chirp source
-  const uint32_t lim = !un.active ? 0u : chirp_in ? nlog + lead : ~0u;
+  if (chirp_in) {
+    // chirp[e] x[e] for e < nlog.  nlog <= M / 2 (M >= 2 nlog - 1 and even), so
+    // the upper half of every unit's elements is zero.  Straight-line loads,
+    // element 0 standing for those past the end: under a mask each element's
+    // chirp was a round trip of its own (first pass of 1 000 003 x 4 40 us).
+    const GlbC<T> *chirp = gc<T>(a.chirp);
+    constexpr int HA = RA / 2;
+    V2<T> ch[HA];
+    const int bm = a.src_mode & 3;
+#pragma unroll
+    for (int j = 0; j < HA; ++j) {
+      const uint32_t e = i + static_cast<uint32_t>(t + RB * j) * tcnt;
+      ch[j] = ldt(chirp, e < nlog ? e : 0u);
+    }
+    if (bm == kSrcComplex) {
+#pragma unroll
+      for (int j = 0; j < HA; ++j) {
+        const uint32_t e = i + static_cast<uint32_t>(t + RB * j) * tcnt;
+        x[j] = ldt(src, lead + (e < nlog ? e : 0u));
+      }
+    } else if (bm == kSrcReal) {
+      const GlbR<T> *rsrc = gr<T>(a.in) + static_cast<int64_t>(un.bq) * a.bs_in;
+#pragma unroll
+      for (int j = 0; j < HA; ++j) {
+        const uint32_t e = i + static_cast<uint32_t>(t + RB * j) * tcnt;
+        x[j] = V2<T>{rsrc[lead + (e < nlog ? e : 0u)], T(0)};
+      }
+    } else {
+      // Hermitian: bins past nlog / 2 are the conjugates of their mirror images,
+      // Im of the bins that are their own dropped
+#pragma unroll
+      for (int j = 0; j < HA; ++j) {
+        const uint32_t e = i + static_cast<uint32_t>(t + RB * j) * tcnt;
+        const uint32_t el = e < nlog ? e : 0u;
+        const bool up = el > nlog / 2;
+        V2<T> v = ldt(src, lead + (up ? nlog - el : el));
+        v.y = (el == 0 || 2 * el == nlog) ? T(0) : up ? -v.y : v.y;
+        x[j] = v;
+      }
+    }
+    const T cs = a.conj_in ? T(-1) : T(1);
+#pragma unroll
+    for (int j = 0; j < HA; ++j) {
+      const uint32_t e = i + static_cast<uint32_t>(t + RB * j) * tcnt;
+      const V2<T> v = cmul(V2<T>{x[j].x, x[j].y * cs}, ch[j]);
+      const bool in = un.active && e < nlog;
+      x[j] = V2<T>{in ? v.x : T(0), in ? v.y : T(0)};
+      x[HA + j] = V2<T>{0, 0};
+    }
+    return;
+  }
+  // a tile that ends partially: idle slots hold zeros
 #pragma unroll
   for (int j = 0; j < RA; ++j) {
     const uint32_t e = ia + static_cast<uint32_t>(t + RB * j) * tcnt;
-    x[j] = e < lim ? ldt(src, e) : V2<T>{0, 0};
+    x[j] = un.active ? ldt(src, e) : V2<T>{0, 0};
   }
 }
 
-// Everything after the loads of tile `blk` (x: what col_load gave).
-// TWM: twiddles from table loads per power (0) or from two or three loads and
-// products (1: w^j = w^(j mod 8) (w^8)^(j / 8), fewer memory instructions).
-// PAIR: the instance also runs the DC / Nyquist pair modes (StageArgs::dc_nyq_pair).
-template <typename T, int C, int RA, int RB, int NCH, int TWM, bool PAIR = false>
-__device__ __forceinline__ void col_rest(const StageArgs &a, int blk, V2<T> (&x)[RA]) {
-  constexpr int R = RA * RB;
-  constexpr int NM = RA / RB;   // stage-B transforms per thread
-  constexpr int KC = RA / NCH;  // k1 values per exchange chunk
-  constexpr int KD = RB / NCH;  // k2 values per block-store chunk
-  constexpr int BL = R / NCH;   // block-store chunk length per unit
-  constexpr int NT = C * RB;
-  static_assert(RA % RB == 0 && RA % NCH == 0 && RB % NCH == 0, "shape");
-  static_assert((C & (C - 1)) == 0, "C must be a power of two");
-  LdsC<T> *lds = lds_base<T>();
-  const int tid = threadIdx.x;
-  const int sl = tid % C;
-  const int t = tid / C;
-  const int64_t u0 = static_cast<int64_t>(blk) * C;
-  const ColUnit un = col_unit<C>(a, blk, sl);
-  const bool active = un.active;
-  const uint32_t bq = un.bq, i = un.i;
-  const bool first = a.p == a.ncol;
-  const uint32_t k = i - fdiv(i, a.fd_p) * static_cast<uint32_t>(a.p);
-  const uint32_t kt = first ? 0u : fdiv(k, a.fd_ncol);
-  const uint32_t tcnt = static_cast<uint32_t>(a.tcnt);
-  const GlbC<T> *tws = gc<T>(a.tw_small);
+// Inter-pass twiddles of the unit's elements: e = t + RB j times w^(e kmul) =
+// w^((t + RB j0) kmul) w^(8 RB jh kmul), j = j0 + 8 jh, from the two-level table.
+template <typename T, int RA, int RB, bool EXACT>
+__device__ __forceinline__ void col_twiddle(const StageArgs &a, uint32_t kmul, int t, V2<T> (&x)[RA]) {
   const GlbC<T> *tw_lo = gc<T>(a.tw_lo);
   const GlbC<T> *tw_hi = gc<T>(a.tw_hi);
   const uint32_t tw_mask = (1u << a.tw_bits) - 1u;
-  const uint32_t kmul = kt * static_cast<uint32_t>(a.twp_mult);
-  const T scale = static_cast<T>(a.scale);
-
-  // ---- input modes of the loaded elements e = t + RB j of the unit -----------
-  // Bluestein chains: the first pass reads chirp[e] x[e] for e < n (zero past
-  // the user length n = nlog), the last passes write conj(X bhat) (forward
-  // chain) or conj(X) chirp for e < n (inverse chain)
-  const bool chirp_in = (a.src_mode & kSrcChirpFlag) != 0;
-  const uint32_t nlog = static_cast<uint32_t>(a.nlog);
-  const GlbC<T> *chirp = gc<T>(a.chirp);
   constexpr int L8 = RA < 8 ? RA : 8;
   constexpr int H8 = (RA + 7) / 8;
-  if (a.conj_in) {
+  auto tw2 = [&](uint32_t mm) __attribute__((always_inline)) {
+    return cmul(ldg(tw_hi + (mm >> a.tw_bits)), ldg(tw_lo + (mm & tw_mask)));
+  };
+  V2<T> blo[8], shi[8];
+  const V2<T> base = tw2(static_cast<uint32_t>(t) * kmul);
+  powers<L8, EXACT, T>([&](int q) __attribute__((always_inline)) { return tw2(static_cast<uint32_t>(RB << q) * kmul); }, blo);
+  powers<H8, EXACT, T>([&](int q) __attribute__((always_inline)) { return tw2(static_cast<uint32_t>((8 * RB) << q) * kmul); }, shi);
+  blo[0] = base;
 #pragma unroll
-    for (int j = 0; j < RA; ++j) x[j].y = -x[j].y;
+  for (int j = 1; j < L8; ++j) blo[j] = cmul(base, blo[j]);
+#pragma unroll
+  for (int j = 0; j < RA; ++j) {
+    const V2<T> w = (j >= 8) ? cmul(blo[j & 7], shi[j >> 3]) : blo[j];
+    x[j] = cmul(x[j], w);
   }
-  if (chirp_in) {
-#pragma unroll
-    for (int j = 0; j < RA; ++j) {
-      const uint32_t e = i + static_cast<uint32_t>(t + RB * j) * tcnt;
-      if (active && e < nlog) x[j] = cmul(x[j], ldt(chirp, e));
-    }
-  }
-  // inter-pass twiddles: element e = t + RB j times w^(e kmul) =
-  // w^((t + RB j0) kmul) w^(8 RB jh kmul), j = j0 + 8 jh, from the two-level table
-  if (!first) {
-    auto tw2 = [&](uint32_t mm) __attribute__((always_inline)) {
-      return cmul(ldg(tw_hi + (mm >> a.tw_bits)), ldg(tw_lo + (mm & tw_mask)));
-    };
-    V2<T> blo[8], shi[H8];
-    if constexpr (TWM == 0) {
-#pragma unroll
-      for (int j = 0; j < L8; ++j) blo[j] = tw2(static_cast<uint32_t>(t + RB * j) * kmul);
-#pragma unroll
-      for (int j = 1; j < H8; ++j) shi[j] = tw2(static_cast<uint32_t>(8 * RB * j) * kmul);
-    } else {
-      const V2<T> base = tw2(static_cast<uint32_t>(t) * kmul);
-      V2<T> sp[8];
-      pow8(tw2(static_cast<uint32_t>(RB) * kmul), sp);
-      blo[0] = base;
-#pragma unroll
-      for (int j = 1; j < L8; ++j) blo[j] = cmul(base, sp[j]);
-      if constexpr (H8 > 1) {
-        shi[1] = tw2(static_cast<uint32_t>(8 * RB) * kmul);
-#pragma unroll
-        for (int j = 2; j < H8; ++j) shi[j] = cmul(shi[j - 1], shi[1]);
-      }
-    }
-#pragma unroll
-    for (int j = 0; j < RA; ++j) {
-      const V2<T> w = (j >= 8) ? cmul(blo[j & 7], shi[j >> 3]) : blo[j];
-      x[j] = cmul(x[j], w);
-    }
-  }
+}
 
+// Both stages of the units' R-point transforms and the transpose between
+// them: x (elements t + RB j) -> y.  bs: y[0] holds k1 = tid % RA of slot tid / RA
+// (two-chunk square instances only), else y[m] holds k1 = t + RB m of slot sl;
+// y[m][k2] is output k1 + RA k2.  Earlier reads of the LDS buffer are done.
+template <typename T, int C, int RA, int RB, int NCH, bool EXACT>
+__device__ __forceinline__ void col_stages(const GlbC<T> *tws, int t, int sl, bool bs, V2<T> (&x)[RA],
+                                           V2<T> (&y)[RA / RB][RB]) {
+  constexpr int NM = RA / RB;   // stage-B transforms per thread
+  constexpr int KC = RA / NCH;  // k1 values per exchange chunk
+  static_assert(RA % RB == 0 && RA % NCH == 0 && RB % NCH == 0, "shape");
+  constexpr int L8 = RA < 8 ? RA : 8;
+  constexpr int H8 = (RA + 7) / 8;
+  LdsC<T> *lds = lds_base<T>();
+  const int tid = threadIdx.x;
   // ---- stage A (radix RA over j) and the inner twiddles ------------------------
   dft<RA>(x);
   // w_R^(t k1) = lo[k1 mod 8] hi[k1 / 8], straight from the length-R table
   // (t k1 < R): two roundings per twiddle
-  V2<T> wlo[8], whi[H8];
-  if constexpr (TWM == 0) {
-#pragma unroll
-    for (int j = 0; j < L8; ++j) wlo[j] = ldt(tws, static_cast<uint32_t>(t * j));
-#pragma unroll
-    for (int j = 0; j < H8; ++j) whi[j] = ldt(tws, static_cast<uint32_t>(t * 8 * j));
-  } else {
-    pow8(ldt(tws, static_cast<uint32_t>(t)), wlo);
-    if constexpr (H8 > 1) {
-      whi[1] = ldt(tws, static_cast<uint32_t>(t * 8));
-#pragma unroll
-      for (int j = 2; j < H8; ++j) whi[j] = cmul(whi[j - 1], whi[1]);
-    }
-  }
+  V2<T> wlo[8], whi[8];
+  powers<L8, EXACT, T>([&](int q) __attribute__((always_inline)) { return ldt(tws, static_cast<uint32_t>(t << q)); }, wlo);
+  powers<H8, EXACT, T>([&](int q) __attribute__((always_inline)) { return ldt(tws, static_cast<uint32_t>((t * 8) << q)); }, whi);
 #pragma unroll
   for (int j = 1; j < RA; ++j) {
     const V2<T> w = (j >= 8) ? ((j & 7) ? cmul(wlo[j & 7], whi[j >> 3]) : whi[j >> 3]) : wlo[j];
@@ -276,7 +283,6 @@ __device__ __forceinline__ void col_rest(const StageArgs &a, int blk, V2<T> (&x)
   }
 
   // ---- RA x RB transpose within each unit and stage B (radix RB over t) -------
-  V2<T> y[NM][RB];
   if constexpr (NCH == 2 && RA == RB) {
     // Two chunks, each holding half of every unit: entry (k1, tt) travels in
     // chunk c = (tt mod 2) xor (k1 >= H).  Every thread writes H values and
@@ -291,7 +297,6 @@ __device__ __forceinline__ void col_rest(const StageArgs &a, int blk, V2<T> (&x)
     // pitch of the chunk buffer keeps either reader at two accesses per bank.
     constexpr int H = RA / 2;
     V2<T> ye[H], yo[H];
-    const bool bs = a.block_store != 0;
     const int pitch = bs ? H * C + 1 : H * C + 8;
     const int rsl = bs ? tid / RA : sl;  // unit slot of this thread's stage-B transform
     const int rk1 = bs ? tid % RA : t;   // and its k1
@@ -330,24 +335,6 @@ __device__ __forceinline__ void col_rest(const StageArgs &a, int blk, V2<T> (&x)
       y[0][k2] = cadd(ye[k2], o);
       y[0][k2 + H] = csub(ye[k2], o);
     });
-    if (bs) {
-      // unit u0 + rsl owns outputs (u0 + rsl) R + e', e' = rk1 + RA k2
-      if (u0 + rsl < a.units) {
-        GlbC<T> *dst = gc<T>(a.out) + u0 * R;
-        const uint32_t o0 = static_cast<uint32_t>(rsl * R + rk1);
-#pragma unroll
-        for (int q = 0; q < RB; ++q) {
-          V2<T> v = y[0][q];
-          if (a.conj_out) v.y = -v.y;
-          if (scale != T(1)) {
-            v.x *= scale;
-            v.y *= scale;
-          }
-          stt(dst, o0 + static_cast<uint32_t>(RA * q), v);
-        }
-      }
-      return;
-    }
   } else {
 #pragma unroll
     for (int c = 0; c < NCH; ++c) {
@@ -367,6 +354,67 @@ __device__ __forceinline__ void col_rest(const StageArgs &a, int blk, V2<T> (&x)
     }
 #pragma unroll
     for (int m = 0; m < NM; ++m) dft<RB>(y[m]);
+  }
+}
+
+// Everything after the loads of tile `blk` (x: what col_load gave).
+template <typename T, int C, int RA, int RB, int NCH, int MODE>
+__device__ __forceinline__ void col_rest(const StageArgs &a, int blk, V2<T> (&x)[RA]) {
+  constexpr int R = RA * RB;
+  constexpr int NM = RA / RB;   // stage-B transforms per thread
+  constexpr int KD = RB / NCH;  // k2 values per block-store chunk
+  constexpr int BL = R / NCH;   // block-store chunk length per unit
+  constexpr int NT = C * RB;
+  static_assert((C & (C - 1)) == 0, "C must be a power of two");
+  LdsC<T> *lds = lds_base<T>();
+  const int tid = threadIdx.x;
+  const int sl = tid % C;
+  const int t = tid / C;
+  const int64_t u0 = static_cast<int64_t>(blk) * C;
+  const ColUnit un = col_unit<C>(a, blk, sl);
+  const bool active = un.active;
+  const uint32_t bq = un.bq, i = un.i;
+  const bool first = a.p == a.ncol;
+  const uint32_t k = i - fdiv(i, a.fd_p) * static_cast<uint32_t>(a.p);
+  const uint32_t kt = first ? 0u : fdiv(k, a.fd_ncol);
+  const uint32_t tcnt = static_cast<uint32_t>(a.tcnt);
+  const uint32_t kmul = kt * static_cast<uint32_t>(a.twp_mult);
+  const T scale = static_cast<T>(a.scale);
+
+  // Bluestein chains: the last passes write conj(X bhat) (forward chain) or
+  // conj(X) chirp for e < n = nlog (inverse chain)
+  const uint32_t nlog = static_cast<uint32_t>(a.nlog);
+  const GlbC<T> *chirp = gc<T>(a.chirp);
+  // (a product, not a branch, which would wait for the data before the
+  // twiddles are on their way; a chirp source is conjugated already)
+  const T cs = (a.conj_in && !(MODE == kColBluestein && (a.src_mode & kSrcChirpFlag))) ? T(-1) : T(1);
+#pragma unroll
+  for (int j = 0; j < RA; ++j) x[j].y *= cs;
+  constexpr bool kExact = RA >= 32 || MODE == kColBluestein;
+  if (!first) col_twiddle<T, RA, RB, kExact>(a, kmul, t, x);
+  V2<T> y[NM][RB];
+  const bool bs = a.block_store != 0;
+  col_stages<T, C, RA, RB, NCH, kExact>(gc<T>(a.tw_small), t, sl, bs, x, y);
+  if constexpr (NCH == 2 && RA == RB) {
+    const int rsl = tid / RA, rk1 = tid % RA;
+    if (bs) {
+      // unit u0 + rsl owns outputs (u0 + rsl) R + e', e' = rk1 + RA k2
+      if (u0 + rsl < a.units) {
+        GlbC<T> *dst = gc<T>(a.out) + u0 * R;
+        const uint32_t o0 = static_cast<uint32_t>(rsl * R + rk1);
+#pragma unroll
+        for (int q = 0; q < RB; ++q) {
+          V2<T> v = y[0][q];
+          if (a.conj_out) v.y = -v.y;
+          if (scale != T(1)) {
+            v.x *= scale;
+            v.y *= scale;
+          }
+          stt(dst, o0 + static_cast<uint32_t>(RA * q), v);
+        }
+      }
+      return;
+    }
   }
 
   auto finish = [&](V2<T> v) __attribute__((always_inline)) {
@@ -415,7 +463,7 @@ __device__ __forceinline__ void col_rest(const StageArgs &a, int blk, V2<T> (&x)
     // forward 2D real column pass with the DC / Nyquist pair in unit 0: its
     // outputs go through LDS so that each thread sees Z_e and Z_-e
     // (workgroup 0 only, uniform over the workgroup)
-    const bool unpack = PAIR && a.dc_nyq_pair == 1 && blk == 0;
+    const bool unpack = MODE == kColPair && a.dc_nyq_pair == 1 && blk == 0;
     if (unpack) {
       __syncthreads();  // the exchange's reads are done
       if (sl == 0) {
@@ -455,22 +503,45 @@ __device__ __forceinline__ void col_rest(const StageArgs &a, int blk, V2<T> (&x)
         auto rel = [&](int m, int q) __attribute__((always_inline)) {
           return static_cast<uint32_t>(t + RB * m + RA * q) * pp;
         };
-        if (a.dst_mode & kDstPointwiseFlag) {
+        // (table loads ahead of the stores in groups: one by one each would
+        // wait for its own round trip)
+        constexpr int G = RB < 16 ? RB : 16;
+        if (MODE == kColBluestein && (a.dst_mode & kDstPointwiseFlag)) {
 #pragma unroll
           for (int m = 0; m < NM; ++m) {
 #pragma unroll
-            for (int q = 0; q < RB; ++q) {
-              const uint32_t o = o0 + rel(m, q);
-              stt(dst, o + lead, cconj(cmul(y[m][q], ldt(bhat, o))));
+            for (int q0 = 0; q0 < RB; q0 += G) {
+              V2<T> w[G];
+#pragma unroll
+              for (int q = 0; q < G; ++q) w[q] = ldt(bhat, o0 + rel(m, q0 + q));
+#pragma unroll
+              for (int q = 0; q < G; ++q) stt(dst, o0 + rel(m, q0 + q) + lead, cconj(cmul(y[m][q0 + q], w[q])));
             }
           }
-        } else if (a.dst_mode & kDstChirpFlag) {
+        } else if (MODE == kColBluestein && (a.dst_mode & kDstChirpFlag)) {
+          // outputs from M / 2 on lie past the user length; a half sink keeps
+          // the bins up to nlog / 2, a real one the real parts
+          const bool real_out = (a.dst_mode & 3) == kDstReal;
+          const uint32_t olim = (a.dst_mode & 3) == kDstHalf ? nlog / 2 + 1 : nlog;
+          GlbR<T> *rdst = gr<T>(a.out) + static_cast<int64_t>(bq) * a.bs_out;
+          constexpr int HB = RB / 2, GB = HB < G ? HB : G;
 #pragma unroll
           for (int m = 0; m < NM; ++m) {
 #pragma unroll
-            for (int q = 0; q < RB; ++q) {
-              const uint32_t o = o0 + rel(m, q);
-              if (o < nlog) stt(dst, o + lead, finish(cmul(cconj(y[m][q]), ldt(chirp, o))));
+            for (int q0 = 0; q0 < HB; q0 += GB) {
+              V2<T> w[GB];
+#pragma unroll
+              for (int q = 0; q < GB; ++q) w[q] = ldt(chirp, min(o0 + rel(m, q0 + q), nlog - 1u));
+#pragma unroll
+              for (int q = 0; q < GB; ++q) {
+                const uint32_t o = o0 + rel(m, q0 + q);
+                const V2<T> v = finish(cmul(cconj(y[m][q0 + q]), w[q]));
+                if (real_out) {
+                  if (o < nlog) rdst[o + lead] = v.x;
+                } else if (o < olim) {
+                  stt(dst, o + lead, v);
+                }
+              }
             }
           }
         } else {
@@ -492,13 +563,76 @@ __device__ __forceinline__ void col_rest(const StageArgs &a, int blk, V2<T> (&x)
   }
 }
 
+// One tile of the middle launch of a two-pass Bluestein convolution M = R0 R
+// (R = RA RA): the forward chain's second pass (p = tcnt = R0), conj(X bhat), and
+// the inverse chain's first pass, which reads the same R elements i + e R0 and
+// writes y[i R + e'].  A square instance leaves its outputs t + RA k2 in the
+// thread that transforms the elements t + RA j next, so the product and the second
+// transform follow in registers.
+template <typename T, int C, int RA, int NCH>
+__device__ __forceinline__ void col_conv_body(const StageArgs &a, int blk) {
+  constexpr int R = RA * RA;
+  const int tid = threadIdx.x;
+  const int sl = tid % C;
+  const int t = tid / C;
+  const int64_t u0 = static_cast<int64_t>(blk) * C;
+  const ColUnit un = col_unit<C>(a, blk, sl);
+  const uint32_t i = un.i, p = static_cast<uint32_t>(a.p);
+  const uint32_t k = i - fdiv(i, a.fd_p) * p;
+  V2<T> x[RA], y[1][RA];
+  col_load<T, C, RA, RA, kColPlain>(a, blk, x);
+  col_twiddle<T, RA, RA, true>(a, k * static_cast<uint32_t>(a.twp_mult), t, x);
+  const GlbC<T> *tws = gc<T>(a.tw_small);
+  col_stages<T, C, RA, RA, NCH, true>(tws, t, sl, false, x, y);
+  const GlbC<T> *bhat = gc<T>(a.bhat);
+  constexpr int G = RA < 16 ? RA : 16;
+#pragma unroll
+  for (int q0 = 0; q0 < RA; q0 += G) {
+    V2<T> w[G];
+#pragma unroll
+    for (int q = 0; q < G; ++q) w[q] = ldt(bhat, i + static_cast<uint32_t>(t + RA * (q0 + q)) * p);
+#pragma unroll
+    for (int q = 0; q < G; ++q) x[q0 + q] = cconj(cmul(y[0][q0 + q], w[q]));
+  }
+  __syncthreads();  // the exchange's reads are done
+  constexpr bool direct = NCH == 2;  // RA-element runs straight from registers
+  col_stages<T, C, RA, RA, NCH, true>(tws, t, sl, direct, x, y);
+  // the tile's units own one contiguous block of C R outputs
+  GlbC<T> *dst = gc<T>(a.out) + u0 * R;
+  const int ns = static_cast<int>(min(static_cast<int64_t>(C), a.units - u0));  // slots with a unit
+  if constexpr (direct) {
+    const int rsl = tid / RA;
+    if (rsl < ns) {
+      const uint32_t o0 = static_cast<uint32_t>(rsl * R + tid % RA);
+#pragma unroll
+      for (int q = 0; q < RA; ++q) stt(dst, o0 + static_cast<uint32_t>(RA * q), y[0][q]);
+    }
+  } else {
+    LdsC<T> *lds = lds_base<T>();
+    constexpr int LSB = (R + R / 32 + 28) / 32 * 32 + 4;
+    __syncthreads();
+#pragma unroll
+    for (int q = 0; q < RA; ++q) {
+      const int e2 = t + RA * q;
+      stc(lds + sl * LSB + e2 + (e2 >> 5), y[0][q]);
+    }
+    __syncthreads();
+#pragma unroll
+    for (int r = 0; r < RA; ++r) {
+      const int f = tid + r * (C * RA);
+      const int s2 = f / R, e2 = f - s2 * R;
+      if (s2 < ns) stt(dst, static_cast<uint32_t>(f), ldc(lds + s2 * LSB + e2 + (e2 >> 5)));
+    }
+  }
+}
+
 // One tile (workgroup `blk` of the launch) of a register-resident pass; every
 // one of the C * RB threads of the workgroup must call it (it synchronises).
-template <typename T, int C, int RA, int RB, int NCH, int TWM, bool PAIR = false>
+template <typename T, int C, int RA, int RB, int NCH, int MODE>
 __device__ __forceinline__ void col_body(const StageArgs &a, int blk) {
   V2<T> x[RA];
-  col_load<T, C, RA, RB, PAIR>(a, blk, x);
-  col_rest<T, C, RA, RB, NCH, TWM, PAIR>(a, blk, x);
+  col_load<T, C, RA, RB, MODE>(a, blk, x);
+  col_rest<T, C, RA, RB, NCH, MODE>(a, blk, x);
 }
 
 }  // namespace dev

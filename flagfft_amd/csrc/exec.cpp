@@ -286,7 +286,11 @@ void Executable::resolve_kernels() {
       case Step::Pass: s.func = pass_kernel(s.dbl, s.ept); break;
       case Step::Leaf: s.func = leaf_kernel(s.dbl, s.leaf_id, s.leaf_mode); break;
       case Step::Stage: s.func = stage_kernel(s.dbl, s.leaf_id, s.leaf_mode); break;
-      case Step::Col: s.func = s.leaf_mode != 0 ? col_pair_kernel(s.leaf_id) : col_kernel(s.leaf_id); break;
+      case Step::Col:
+        s.func = s.leaf_mode == 2   ? col_conv_kernel(s.leaf_id)
+                 : s.leaf_mode == 1 ? col_pair_kernel(s.leaf_id)
+                                    : col_kernel(s.leaf_id, s.leaf_mode == 3);
+        break;
       case Step::Mfma: s.func = mfma_kernel(s.compute, s.leaf_id); break;
       case Step::BluesteinLds: s.func = bluestein_lds_kernel(s.leaf_id, s.leaf_mode); break;
       case Step::BluesteinCombine: s.func = bluestein_combine_kernel(s.dbl, s.split); break;
@@ -834,12 +838,15 @@ bool Builder::try_stage(const PassArgs &a, const std::vector<int> &radices, int 
   // register-resident two-stage pass (plain complex passes, and Bluestein
   // chain ends: chirp source, pointwise and chirp sinks)
   const bool col_allowed = mode == 0 && opt_.stage_form != 2 && (!opt_.generic_kernels || opt_.queue_form) &&
-                           (a.src_mode & 3) == kSrcComplex && (a.dst_mode & 3) == kDstComplex;
-  int cid = !col_allowed        ? -1
+                           ((a.src_mode & 3) == kSrcComplex || (a.src_mode & kSrcChirpFlag)) &&
+                           ((a.dst_mode & 3) == kDstComplex || (a.dst_mode & kDstChirpFlag));
+  const bool conv_allowed = mode == 1 && opt_.stage_form != 2 && !opt_.generic_kernels && opt_.forced_units == 0;
+  int cid = conv_allowed        ? col_conv_kernel_id(a.R, dbl(), a.units)
+            : !col_allowed      ? -1
             : opt_.queue_form ? col_queue_kernel_id(a.R, dbl())
             : opt_.forced_units != 0
                 ? col_kernel_id(a.R, dbl(), opt_.forced_units, a.p == 1)
-                : col_kernel_id_for(a.R, dbl(), a.p == 1, a.units);
+                : col_kernel_id_for(a.R, dbl(), a.p == 1, a.units, !s.col_fast);
   // DC / Nyquist pair: one transform's single column pass over the n1 / 2
   // columns of the half spectrum (row pitch n1 / 2 + 1) but its Nyquist
   // column, which goes with column 0; the other side is a workspace of n1 / 2
@@ -853,9 +860,12 @@ bool Builder::try_stage(const PassArgs &a, const std::vector<int> &radices, int 
     cid = col_pair_kernel_id(a.R, dbl());
     if (cid < 0) throw std::logic_error("DC/Nyquist pair: no paired column instance");
   }
-  if ((sid < 0 && cid < 0) || (a.src_mode & 3) != kSrcComplex || (a.dst_mode & 3) != kDstComplex) return false;
+  // (the LDS super-stage reads and writes complex sequences only)
+  const bool complex_ends = (a.src_mode & 3) == kSrcComplex && (a.dst_mode & 3) == kDstComplex;
+  if ((sid < 0 && cid < 0) || (cid < 0 && !complex_ends)) return false;
   // contiguous sequences, or the columns of contiguous rows of ncol elements
   const bool rows = !s.col_fast && s.ncol == 1 && a.gi.es == 1 && a.go.es == 1;
+  if (mode == 1 && a.go.bs != n) throw std::runtime_error("convolution pass needs contiguous sequences");
   const bool cols = pair || (s.col_fast && s.ncol > 1 && a.gi.es == s.ncol && a.gi.cs == 1 && a.go.es == s.ncol &&
                              a.go.cs == 1 && mode == 0 && a.src_mode == kSrcComplex && a.dst_mode == kDstComplex);
   if (!rows && !cols) return false;
@@ -873,7 +883,7 @@ bool Builder::try_stage(const PassArgs &a, const std::vector<int> &radices, int 
   const bool col_ok =
       cid >= 0 && col_tiles_fit(tcnt, p, R, cunits, a.gi.bs, a.go.bs, pair ? 1 : units / tcnt, eb());
   if (pair && !col_ok) throw std::logic_error("DC/Nyquist pair: the column pass does not fit");
-  if (!col_ok && sid < 0) return false;
+  if (!col_ok && (sid < 0 || !complex_ends)) return false;
   if (col_ok) {
     Step cst;
     cst.kind = Step::Col;
@@ -899,7 +909,7 @@ bool Builder::try_stage(const PassArgs &a, const std::vector<int> &radices, int 
     g.conj_out = a.conj_out;
     g.scale = a.scale;
     g.units = units;
-    g.block_store = (rows && p == 1 && a.go.bs == n && a.dst_mode == kDstComplex) ? 1 : 0;
+    g.block_store = (mode == 1 || (rows && p == 1 && a.go.bs == n && a.dst_mode == kDstComplex)) ? 1 : 0;
     g.src_mode = a.src_mode;
     g.dst_mode = a.dst_mode;
     g.nlog = a.nlog;
@@ -910,6 +920,8 @@ bool Builder::try_stage(const PassArgs &a, const std::vector<int> &radices, int 
       cst.leaf_mode = 1;  // the paired instance (Executable::resolve_kernels)
       ++pair_steps_;
     }
+    if (mode == 1) cst.leaf_mode = 2;  // the convolution launch
+    if (mode == 0 && (a.src_mode != kSrcComplex || a.dst_mode != kDstComplex)) cst.leaf_mode = 3;  // Bluestein ends
     const int64_t nblocks = (g.units + cunits - 1) / cunits;
     g.nblocks = static_cast<int32_t>(nblocks);
     g.xcd_remap = opt_.xcd_remap;
@@ -919,8 +931,11 @@ bool Builder::try_stage(const PassArgs &a, const std::vector<int> &radices, int 
     cst.bytes_moved = s.nbatch * (pair ? units + 1 : ncol) *
                       (src_bytes(a.src_mode, n, a.nlog, eb()) + dst_bytes(a.dst_mode, n, a.nlog, eb()));
     std::ostringstream lab;
-    lab << "k_col<" << (dbl() ? "fp64" : "fp32") << "," << col_kernel_targs(cid, pair) << "> pass " << pass << "/"
-        << npasses << " R=" << R << " p=" << p << " tcnt=" << tcnt << (g.block_store ? " block-store" : "")
+    if (mode == 1)
+      lab << "k_col_conv<" << (dbl() ? "fp64" : "fp32") << "," << col_conv_targs(cid) << "> convolution ";
+    else
+      lab << "k_col<" << (dbl() ? "fp64" : "fp32") << "," << col_kernel_targs(cid, cst.leaf_mode == 3 ? 2 : cst.leaf_mode) << "> pass ";
+    lab << pass << "/" << npasses << " R=" << R << " p=" << p << " tcnt=" << tcnt << (g.block_store ? " block-store" : "")
         << (cols ? " columns=" : "");
     if (cols) lab << ncol;
     if (pair) lab << (pair_ == 1 ? " dc-nyquist-unpack" : " dc-nyquist-pack");
@@ -961,7 +976,6 @@ bool Builder::try_stage(const PassArgs &a, const std::vector<int> &radices, int 
   g.scale = a.scale;
   g.units = a.units;
   g.block_store = (mode == 1 || (rows && p == 1 && a.dst_mode == kDstComplex && a.go.bs == n)) ? 1 : 0;
-  if (mode == 1 && a.go.bs != n) throw std::runtime_error("convolution pass needs contiguous sequences");
   g.src_mode = a.src_mode;
   g.dst_mode = a.dst_mode;
   g.nlog = a.nlog;
@@ -1252,6 +1266,23 @@ void Builder::emit_bluestein_split(const Core &c, const SeqSet &s, int src, int 
   ex_.steps.push_back(cb);
 }
 
+// Whether the outer launches of a two-pass Bluestein convolution of length M
+// with super-radix r0 run on register-resident instances for these sequences.
+bool Builder::conv_ends_in_registers(int64_t r0, int64_t M, const SeqSet &s) {
+  if (opt_.stage_form == 2 || opt_.forced_units != 0) return false;
+  const int64_t tcnt = M / r0;
+  for (bool first : {true, false}) {
+    const int id = col_kernel_id_for(r0, dbl(), first, s.nbatch * tcnt, true);
+    int units = 0, threads = 0, ebytes = 0;
+    size_t lds = 0;
+    if (id < 0) return false;
+    col_kernel_shape(id, units, threads, lds, ebytes);
+    if (!col_tiles_fit(tcnt, tcnt, static_cast<int>(r0), units, std::max(s.gi.bs, M), std::max(s.go.bs, M), s.nbatch, eb()))
+      return false;
+  }
+  return true;
+}
+
 void Builder::emit_bluestein(const Core &c, const SeqSet &s, int src, int dst, const Modes &m) {
   const int64_t n = c.n, M = c.m;
   if (c.lds_conv) {
@@ -1343,9 +1374,11 @@ void Builder::emit_bluestein(const Core &c, const SeqSet &s, int src, int dst, c
     ex_.steps.push_back(st);
     return;
   }
+  // (real and Hermitian sequences: the register-resident outer passes only)
+  const bool complex_ends = (m.src_mode & 3) == kSrcComplex && (m.dst_mode & 3) == kDstComplex;
   if (c.conv && c.conv->passes.size() == 2 && !opt_.generic_kernels && !s.col_fast && s.ncol == 1 &&
-      s.gi.es == 1 && s.go.es == 1 && (m.src_mode & 3) == kSrcComplex && (m.dst_mode & 3) == kDstComplex &&
-      stage_kernel_id(c.conv->pass_radices[0]) >= 0 && stage_kernel_id(c.conv->pass_radices[1]) >= 0) {
+      s.gi.es == 1 && s.go.es == 1 && conv_passes_compiled(c.conv->passes[0], c.conv->passes[1], prec_, opt_) &&
+      (complex_ends || conv_ends_in_registers(c.conv->passes[0], M, s))) {
     // Three launches over M = R0 * R1:
     //   A  chirp * x, forward pass 0 (R0)                        user -> wA
     //   B  forward pass 1 (R1), conj(X * bhat), inverse pass 0 (R1, the

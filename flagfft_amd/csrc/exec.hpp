@@ -212,6 +212,7 @@ class Builder {
                       std::initializer_list<int> avoid_extra);
   void emit_rader(const Core &c, const SeqSet &s, int src, int dst, const Modes &m);
   void emit_bluestein(const Core &c, const SeqSet &s, int src, int dst, const Modes &m);
+  bool conv_ends_in_registers(int64_t r0, int64_t M, const SeqSet &s);
   void emit_bluestein_split(const Core &c, const SeqSet &s, int src, int dst, const Modes &m, int split);
   bool try_leaf_split(const Core &c, const SeqSet &s, int src, int dst, const Modes &m);
   bool try_leaf_split_real(const Plan1D &pl, const SeqSet &s, int src, int dst);

@@ -737,7 +737,7 @@ __global__ __launch_bounds__(kQueueThreads) __attribute__((amdgpu_waves_per_eu(W
 #pragma unroll
     for (int w = 0; w < NW; ++w) u.w[w] = __builtin_amdgcn_readlane(mine, w);
     const int first = __builtin_amdgcn_readfirstlane(q.jobs[lo].first);
-    col_body<T, C, RA, RB, NCH, 1>(u.a, item - first);
+    col_body<T, C, RA, RB, NCH, kColBluestein>(u.a, item - first);
   }
 }
 

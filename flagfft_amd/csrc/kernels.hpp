@@ -42,6 +42,7 @@ const void *leaf_kernel(bool dbl, int id, int mode);  // mode: 0 complex, 1 R2C,
 // Specialised super-stage kernels: id of the compiled radix sequence (-1 if none),
 // its units per workgroup and elements per thread.
 int stage_kernel_id(const std::vector<int> &radices);
+std::vector<int64_t> stage_kernel_radices();  // the super-radices of all instances
 // The instance with `units` per workgroup (0: the default one), -1 if none.
 int stage_kernel_id(const std::vector<int> &radices, bool dbl, int units);
 void stage_kernel_shape(int id, bool dbl, int &units_per_group, int &ept);
@@ -55,17 +56,19 @@ bool stage_kernel_fast(int id);
 // its units, threads, dynamic LDS bytes and element bytes; the kernel.
 int col_kernel_id(int64_t r, bool dbl, int units);
 int col_kernel_id(int64_t r, bool dbl, int units, bool first);
-// The default instance for a launch of total_units units: a narrower tile when
+// The default instance for a launch of total_units units (rows: of contiguous
+// sequences, not columns): a narrower tile when
 // the default one would leave CUs without a workgroup, -1 where the LDS
 // super-stage is faster for so few.
-int col_kernel_id_for(int64_t r, bool dbl, bool first, int64_t total_units);
+int col_kernel_id_for(int64_t r, bool dbl, bool first, int64_t total_units, bool rows);
 // Row-segment bytes (units x element bytes) of the default instance, 0 if none.
 int col_run_bytes(int64_t r, bool dbl, bool first);
 // Whether the tile of some instance of radix r divides tcnt units.
 bool col_tiles_divide(int64_t r, bool dbl, int64_t tcnt);
 int col_kernel_radix(int id);
+std::vector<int64_t> col_kernel_radices(bool dbl);  // the super-radices of all instances
 void col_kernel_shape(int id, int &units, int &threads, size_t &lds_bytes, int &elem_bytes);
-const void *col_kernel(int id);
+const void *col_kernel(int id, bool bluestein);  // bluestein: with the modes of Bluestein chain ends
 // The same instance with the DC / Nyquist pair modes of a 2D real column pass
 // (StageArgs::dc_nyq_pair), null if it has none; the first-pass default
 // instance of r when it has one, else -1.
@@ -75,8 +78,13 @@ int col_pair_kernel_id(int64_t r, bool dbl);
 // none for r), and its queue variant (QueueJob::variant; -1 for others).
 int col_queue_kernel_id(int64_t r, bool dbl);
 int col_queue_variant(int id);
+// The instance whose convolution launch (k_col_conv) a Bluestein chain of
+// total_units units runs, -1 if none for r; its kernel and template arguments.
+int col_conv_kernel_id(int64_t r, bool dbl, int64_t total_units);
+const void *col_conv_kernel(int id);
+std::string col_conv_targs(int id);
 // Template arguments after the element type, as the kernel symbol lists them.
-std::string col_kernel_targs(int id, bool pair = false);
+std::string col_kernel_targs(int id, int mode);  // mode: ColMode
 
 // Persistent mixed-length kernel (kQueueThreads threads per workgroup, one
 // QueueArgs argument).

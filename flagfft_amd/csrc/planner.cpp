@@ -252,6 +252,82 @@ bool cheapest_split(int64_t n, Prec p, const PlanOptions &o, std::vector<int64_t
   return have;
 }
 
+void chain_core(int64_t n, const std::vector<int64_t> &passes, Core &c) {
+  c.kind = CoreKind::MultiPass;
+  c.n = n;
+  c.passes = passes;
+  c.pass_radices.clear();
+  for (int64_t r : passes) {
+    std::vector<int> rad;
+    radix_factor(r, rad);
+    c.pass_radices.push_back(rad);
+  }
+}
+
+// Relative time per element of the convolution pass of super-radix r: its
+// sweep and two transforms; 0 if no kernel.  Square register-resident
+// instances run at about 3.3 TB/s (4096 points: 1.9), LDS super-stages at 2.2,
+// their 5- and 10-smooth instances at 0.9.
+double conv_time(int64_t r, Prec p, const PlanOptions &o) {
+  if (o.stage_form != 2 && o.forced_units == 0 && col_conv_kernel_id(r, p == Prec::F64, 0) >= 0)
+    return r >= 4096 ? 1.0 / 1.9 : 1.0 / 3.3;
+  std::vector<int> rad;
+  if (!radix_factor(r, rad)) return 0.0;
+  const int id = stage_kernel_id(rad);
+  return id < 0 ? 0.0 : stage_kernel_fast(id) ? 1.0 / 2.2 : 1.0 / 0.9;
+}
+
+// Two-pass Bluestein convolutions M = R0 R1 in three launches, over the
+// super-radices with a compiled kernel, by the time of the launches (the outer
+// ones read or write the user's n <= M / 2 elements on one side).
+class ConvSplits {
+ public:
+  ConvSplits(Prec p, const PlanOptions &o) {
+    const int64_t cap = pass_max(o, p);
+    const bool col_ok = o.stage_form != 2 && o.forced_units == 0;
+    std::vector<int64_t> all = stage_kernel_radices();
+    for (int64_t r : col_kernel_radices(p == Prec::F64)) all.push_back(r);
+    std::sort(all.begin(), all.end(), std::greater<int64_t>());
+    all.erase(std::unique(all.begin(), all.end()), all.end());
+    for (int64_t r : all) {
+      std::vector<int> rad;
+      if (r > cap || !radix_factor(r, rad)) continue;
+      Radix x{r, 0.0, conv_time(r, p, o)};
+      const int sid = stage_kernel_id(rad);
+      if (col_ok && col_kernel_id(r, p == Prec::F64, 0) >= 0)
+        x.outer = pass_time(r, p, true, o, 0) + pass_time(r, p, false, o, 0);
+      else if (sid >= 0)
+        x.outer = 2.0 / (stage_kernel_fast(sid) ? 2.6 : 1.2);  // an LDS super-stage with the chirp at either end
+      if (x.outer > 0.0 || x.conv > 0.0) rs_.push_back(x);
+    }
+  }
+  // The split of the cheapest M = R0 R1 in [lo, hi] (false: none).
+  bool best(int64_t lo, int64_t hi, std::vector<int64_t> &split) const {
+    double best_t = 0.0;
+    for (const Radix &x1 : rs_) {
+      if (x1.conv == 0.0) continue;
+      for (const Radix &x0 : rs_) {
+        const int64_t M = x0.r * x1.r;
+        if (x0.outer == 0.0 || M < lo || M > hi) continue;
+        const double tt = (0.75 * x0.outer + x1.conv) * static_cast<double>(M);
+        if (best_t == 0.0 || tt < best_t * 0.98 ||
+            (tt <= best_t * 1.02 && std::min(x0.r, x1.r) > std::min(split[0], split[1]))) {
+          split = {x0.r, x1.r};
+          best_t = tt;
+        }
+      }
+    }
+    return best_t > 0.0;
+  }
+
+ private:
+  struct Radix {
+    int64_t r;
+    double outer, conv;  // time as R0 / as R1, 0: no kernel
+  };
+  std::vector<Radix> rs_;
+};
+
 bool multipass_core(int64_t n, Prec p, const PlanOptions &o, Core &c, bool by_cost = false) {
   std::vector<int64_t> passes;
   const int64_t cap = pass_max(o, p);
@@ -272,15 +348,7 @@ bool multipass_core(int64_t n, Prec p, const PlanOptions &o, Core &c, bool by_co
   if (!ok && by_cost) ok = cheapest_split(n, p, o, passes);
   for (int k = 2; !ok && k <= 4; ++k) ok = split_passes(n, k, cap, passes);
   if (!ok) return false;
-  c.kind = CoreKind::MultiPass;
-  c.n = n;
-  c.passes = passes;
-  c.pass_radices.clear();
-  for (int64_t r : passes) {
-    std::vector<int> rad;
-    radix_factor(r, rad);
-    c.pass_radices.push_back(rad);
-  }
+  chain_core(n, passes, c);
   return true;
 }
 
@@ -291,6 +359,13 @@ int rader_lds_bytes(int64_t p, Prec prec) {
 }
 
 }  // namespace
+
+bool conv_passes_compiled(int64_t r0, int64_t r1, Prec p, const PlanOptions &o) {
+  std::vector<int> rad;
+  if (!radix_factor(r0, rad)) return false;
+  const bool col = o.stage_form != 2 && o.forced_units == 0 && col_kernel_id(r0, p == Prec::F64, 0) >= 0;
+  return (col || stage_kernel_id(rad) >= 0) && conv_time(r1, p, o) > 0.0;
+}
 
 Core plan_core(int64_t n, Prec p, const PlanOptions &o) {
   if (n < 1) throw std::invalid_argument("transform length must be positive");
@@ -332,10 +407,11 @@ Core plan_core(int64_t n, Prec p, const PlanOptions &o) {
     }
   }
   if (smooth19(n) && multipass_core(n, p, o, c, true)) return c;
-  // Bluestein over a 13-smooth convolution length M >= 2n-1.  A length that
-  // fits one LDS pass is taken as soon as it is found (the whole convolution
-  // is one launch).  Otherwise every M up to twice the minimum is weighed by
-  // its HBM sweeps: M x passes, x 2.5 when a pass has no fast specialised
+  // Bluestein over a 13-smooth convolution length M >= 2n-1: the first that
+  // fits one LDS pass (the whole convolution is one launch), else the two-pass M
+  // up to twice the minimum with the cheapest three launches (ConvSplits).
+  // Lengths past those, explicit splits and persistent-queue plans weigh every
+  // M by its HBM sweeps: M x passes, x 2.5 when a pass has no fast specialised
   // kernel (the run-time-radix pass and the 5- / 10-smooth instances run
   // about that much slower than the power-of-two passes).
   Core best;
@@ -358,6 +434,15 @@ Core plan_core(int64_t n, Prec p, const PlanOptions &o) {
       c.lds_halves = pick->halves;
       return c;
     }
+  }
+  std::vector<int64_t> split;
+  if (m0 > lmax && o.forced_passes.empty() && !o.generic_kernels && ConvSplits(p, o).best(m0, 2 * m0 + 64, split)) {
+    c.kind = CoreKind::Bluestein;
+    c.m = split[0] * split[1];
+    c.radices.clear();
+    c.conv = std::make_shared<Core>();
+    chain_core(c.m, split, *c.conv);
+    return c;
   }
   for (int64_t M = m0;; ++M) {
     if (have && static_cast<double>(M) >= best_cost) break;

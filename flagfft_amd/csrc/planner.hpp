@@ -117,6 +117,9 @@ int col_kernel_id_dividing(int64_t r, bool dbl, int64_t tcnt);
 bool passes_specialised(const std::vector<int64_t> &passes, bool fast_only = false);
 bool stage_kernel_fast(int id);
 
+// Whether the three launches of a two-pass Bluestein convolution R0 * R1 have
+// specialised kernels (R0: chain passes, R1: the convolution pass).
+bool conv_passes_compiled(int64_t r0, int64_t r1, Prec p, const PlanOptions &o);
 Core plan_core(int64_t n, Prec p, const PlanOptions &o);
 PlanTree plan_tree(const PlanDesc &d, const PlanOptions &o);
 

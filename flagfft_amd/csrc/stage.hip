@@ -235,6 +235,16 @@ int stage_kernel_id(const std::vector<int> &radices, bool dbl, int units) {
 
 int stage_kernel_id(const std::vector<int> &radices) { return stage_kernel_id(radices, false, 0); }
 
+std::vector<int64_t> stage_kernel_radices() {
+  std::vector<int64_t> v;
+  for (const StageEntry &e : kStageTable) {
+    int64_t r = 1;
+    for (int j = 0; j < e.nrad; ++j) r *= e.rad[j];
+    v.push_back(r);
+  }
+  return v;
+}
+
 bool stage_kernel_fast(int id) { return kStageTable[id].fast; }
 
 void stage_kernel_shape(int id, bool dbl, int &units_per_group, int &ept) {
