@@ -113,6 +113,87 @@ const ColEntry kColTable[] = {
 
 }  // namespace
 
+namespace {
+
+// Passes fused with the split-spectrum pass of a real transform, per super-radix
+// in order of falling tile: half a tile's row segment is its mirror units', so the
+// tiles are twice as wide as the plain passes' where they fit.  The narrow ones
+// serve launches that leave CUs idle otherwise.  Two workgroups per CU of the wide
+// tiles hide the exchanges (WPE 4; the 512-point one spills 10 VGPRs so and is still
+// faster: 2^20 x 16 R2C 68.3 us, 70.4 without).
+//
+// Times of whole R2C / C2R transforms, with a pass of its own -> fused: 2^20 x 16
+// 78 -> 68 / 83 -> 60 us, 65536 x 512 R2C 157 -> 102, 2^20 x 1 27.5 -> 18.7 / 28.3 -> 19.1,
+// 2^17 x 8 R2C 19.7 -> 11.5, 2^22 x 4 97 -> 74 / 89 -> 61, FP64 2^20 x 8 93 -> 66 / 86 -> 55.
+// Odd row lengths h + 1 misalign the runs of R2C stores, so those cannot bypass the
+// caches (non-temporal stores: 68 -> 78 us), and the next transform's first pass
+// shares HBM with their write-back.
+struct ColRealEntry {
+  int r, ra, rb, c;
+  bool dbl;
+  const void *post, *pre;
+};
+#define FLAGFFT_COLR(T, C, RA, RB, NCH, WPE)                                              \
+  {RA * RB, RA, RB, C, sizeof(T) == 8,                                                    \
+   (const void *)dev::k_col<T, C, RA, RB, NCH, WPE, dev::kColRealPost>,                   \
+   (const void *)dev::k_col<T, C, RA, RB, NCH, WPE, dev::kColRealPre>}
+const ColRealEntry kColRealTable[] = {
+    FLAGFFT_COLR(float, 16, 64, 32, 2, 2),   // 2048
+    FLAGFFT_COLR(float, 32, 32, 32, 2, 4),   // 1024
+    FLAGFFT_COLR(float, 8, 32, 32, 2, 4),
+    FLAGFFT_COLR(float, 32, 32, 16, 2, 4),   // 512
+    FLAGFFT_COLR(float, 8, 32, 16, 2, 2),
+    FLAGFFT_COLR(float, 32, 16, 16, 1, 4),   // 256
+    FLAGFFT_COLR(float, 8, 16, 16, 1, 4),
+    FLAGFFT_COLR(float, 32, 16, 8, 1, 4),    // 128
+    FLAGFFT_COLR(float, 64, 8, 8, 1, 4),     // 64
+    FLAGFFT_COLR(double, 8, 32, 32, 2, 2),   // 1024
+    FLAGFFT_COLR(double, 16, 32, 16, 2, 2),  // 512
+    FLAGFFT_COLR(double, 16, 16, 16, 1, 4),  // 256
+    FLAGFFT_COLR(double, 4, 16, 16, 1, 4),
+    FLAGFFT_COLR(double, 16, 16, 8, 1, 4),   // 128
+    FLAGFFT_COLR(double, 32, 8, 8, 1, 4),    // 64
+};
+
+}  // namespace
+
+int col_real_kernel_id(int64_t r, bool dbl, int64_t tcnt, int64_t total_units) {
+  int best = -1, bc = 0;
+  for (int id = 0; id < static_cast<int>(sizeof(kColRealTable) / sizeof(kColRealTable[0])); ++id) {
+    const ColRealEntry &e = kColRealTable[id];
+    if (e.r != r || e.dbl != dbl || tcnt % e.c != 0) continue;
+    if (best < 0 || total_units < static_cast<int64_t>(kColGroups) * bc) {
+      best = id;
+      bc = e.c;
+    }
+  }
+  // 2048 points once CUs run dry (2^22 x 1 C2R: 45 us, 37 with the pass of its own)
+  if (r == 2048 && total_units < static_cast<int64_t>(kColGroups) * bc) return -1;
+  return best;
+}
+
+void col_real_kernel_shape(int id, int &units, int &threads, size_t &lds_bytes, int &elem_bytes) {
+  const ColRealEntry &e = kColRealTable[id];
+  units = e.c;
+  threads = e.c * e.rb;
+  elem_bytes = e.dbl ? 16 : 8;
+  const int half = e.ra / 2 * e.rb * e.c;  // the mirror exchange; the two-chunk forms' exchange and block store
+  int need = half + half / 32;
+  if (e.ra == 32 && e.rb == 32) need = std::max(need, e.ra * ((e.ra / 2) * e.c + 8));
+  const int nch = e.ra >= 32 ? 2 : 1;
+  const int ex = e.ra / nch * e.rb * e.c;
+  const int bl = e.r / nch;
+  need = std::max({need, ex + (ex >> 5) + 1, e.c * ((bl + bl / 32 + 28) / 32 * 32 + 4)});
+  lds_bytes = static_cast<size_t>(need) * static_cast<size_t>(elem_bytes);
+}
+
+const void *col_real_kernel(int id, bool post) { return post ? kColRealTable[id].post : kColRealTable[id].pre; }
+
+std::string col_real_targs(int id, bool post) {
+  const ColRealEntry &e = kColRealTable[id];
+  return std::to_string(e.c) + "," + std::to_string(e.ra) + "," + std::to_string(e.rb) + (post ? ",post" : ",pre");
+}
+
 // units: 0 for the default instance of a first (first = true) or later
 // pass, C for the first instance with C units per workgroup, 1000 NCH + C
 // for the one with NCH exchange chunks as well.

@@ -81,7 +81,11 @@ __device__ __forceinline__ void powers(Get get, V2<T> *p) {
 // source, pointwise and chirp sinks).  Instances of their own: the sinks' table
 // values cost the 64 x 256-point pass its second workgroup per CU (42 -> 54 us of
 // 65536 x 256).
-enum ColMode : int { kColPlain = 0, kColPair = 1, kColBluestein = 2 };
+//
+// kColRealPost / kColRealPre: the last / first pass of the n/2-point chain of an
+// even-length real transform, with the split-spectrum pass in it (real_partner):
+// a tile holds C / 2 units and their mirror units.
+enum ColMode : int { kColPlain = 0, kColPair = 1, kColBluestein = 2, kColRealPost = 3, kColRealPre = 4 };
 
 // Unit slot `sl` of tile `blk`: its position i in sequence bq + dq, where bq
 // is the sequence of the tile's first unit (uniform over the workgroup: the
@@ -96,9 +100,26 @@ struct ColUnit {
   bool active;  // the slot has a unit
   bool whole;   // every slot of the tile has one (uniform)
 };
+// Unit of slot sl of a real tile whose first pair is j0.
 template <int C>
+__device__ __forceinline__ uint32_t pair_unit(uint32_t j0, uint32_t tcnt, int sl) {
+  const uint32_t j = j0 + static_cast<uint32_t>(sl % (C / 2));
+  return sl < C / 2 ? j : j == 0 ? tcnt / 2 : tcnt - j;
+}
+template <int C, int MODE>
 __device__ __forceinline__ ColUnit col_unit(const StageArgs &a, int blk, int sl) {
   const uint32_t u0 = static_cast<uint32_t>(blk) * C;
+  if constexpr (MODE == kColRealPost || MODE == kColRealPre) {
+    // whole tiles of one sequence: units j and tcnt - j (0 and tcnt / 2 are their
+    // own mirror units and share the pair j = 0)
+    ColUnit r;
+    const uint32_t tcnt = static_cast<uint32_t>(a.tcnt);
+    r.bq = fdiv(u0, a.fd_tcnt);
+    r.dq = 0;
+    r.i = pair_unit<C>((u0 - r.bq * tcnt) / 2, tcnt, sl);
+    r.active = r.whole = true;
+    return r;
+  }
   const uint32_t units = static_cast<uint32_t>(a.units);
   const uint32_t u = min(u0 + static_cast<uint32_t>(sl), units - 1u);
   ColUnit r;
@@ -118,7 +139,7 @@ __device__ __forceinline__ void col_load(const StageArgs &a, int blk, V2<T> (&x)
   const int tid = threadIdx.x;
   const int sl = tid % C;
   const int t = tid / C;
-  const ColUnit un = col_unit<C>(a, blk, sl);
+  const ColUnit un = col_unit<C, MODE>(a, blk, sl);
   const uint32_t i = un.i;
   const uint32_t tcnt = static_cast<uint32_t>(a.tcnt);
   const uint32_t lead = un.dq * static_cast<uint32_t>(a.bs_in);
@@ -357,6 +378,59 @@ __device__ __forceinline__ void col_stages(const GlbC<T> *tws, int t, int sl, bo
   }
 }
 
+// Split-spectrum pass of a real transform on the elements m = i + e np of a tile
+// of unit pairs: thread t holds e = t + RB q in v[q]; the mirror bin h - m
+// (h = np R) is element R - 1 - e of the mirror unit np - i, so v[RA - 1 - q] of thread
+// RB - 1 - t in the other half of the tile (unit 0 mirrors e into R - e of itself,
+// unit np / 2 into R - 1 - e of itself).  The values change places through LDS in two
+// halves; v[q] becomes combine(q, v[q], mirror value, own): own where the bin is
+// its own mirror (bins 0 and h / 2, whose mirror value given is v[q] itself).
+//
+// In a pass of its own the bins are read and written once more (67 MB each way of
+// 2^20 x 16 R2C, 22-37 us of 75-93).
+template <typename T, int C, int RA, int RB, typename F>
+__device__ __forceinline__ void real_partner(uint32_t i, uint32_t np, int t, int sl, V2<T> (&v)[RA], F combine) {
+  constexpr int HQ = RA / 2;
+  static_assert(RB * C % 32 == 0, "padding");
+  LdsC<T> *lds = lds_base<T>();
+  const bool own_unit = i == 0 || 2 * i == np;
+  const int pt = i != 0 ? RB - 1 - t : t == 0 ? 0 : RB - t;
+  const int ps = own_unit ? sl : sl ^ (C / 2);
+  const bool wrap = i == 0 && t == 0;  // q mirrors into RA - q
+  const int b0 = pt * C + ps;
+  const int b1 = wrap ? b0 + RB * C : b0;
+  const LdsC<T> *r0 = lds + b0 + (b0 >> 5), *r1 = lds + b1 + (b1 >> 5);
+  constexpr int row = RB * C + RB * C / 32;
+  V2<T> up[HQ];
+#pragma unroll
+  for (int c = 0; c < 2; ++c) {
+    __syncthreads();  // earlier reads of the buffer are done
+#pragma unroll
+    for (int qq = 0; qq < HQ; ++qq) stc(lds + xslot<C, RB>(qq, t, sl), v[c * HQ + qq]);
+    __syncthreads();
+    sfor<HQ>([&](auto Q) __attribute__((always_inline)) {
+      constexpr int qq = decltype(Q)::value;
+      // the first of a half wraps past the buffer: those bins are their own mirror
+      const V2<T> m = ldc((qq == 0 ? r0 : r1) + (HQ - 1 - qq) * row);
+      if (c == 0) {
+        up[qq] = m;
+      } else {
+        const bool own = qq == 0 && wrap;
+        v[qq] = combine(std::integral_constant<int, qq>{}, v[qq], own ? v[qq] : m, own);
+        v[HQ + qq] = combine(std::integral_constant<int, HQ + qq>{}, v[HQ + qq], own ? v[HQ + qq] : up[qq], own);
+      }
+    });
+  }
+}
+
+// w_n^(i + t np) of the first element of a thread; element t + RB q has
+// w_2RA^q times that (n = 2 np RA RB).
+template <typename T>
+__device__ __forceinline__ V2<T> real_twiddle(const StageArgs &a, uint32_t i, uint32_t np, int t) {
+  const uint32_t m = i + static_cast<uint32_t>(t) * np;
+  return cmul(ldg(gc<T>(a.tw_rhi) + (m >> a.tw_rbits)), ldg(gc<T>(a.tw_rlo) + (m & ((1u << a.tw_rbits) - 1u))));
+}
+
 // Everything after the loads of tile `blk` (x: what col_load gave).
 template <typename T, int C, int RA, int RB, int NCH, int MODE>
 __device__ __forceinline__ void col_rest(const StageArgs &a, int blk, V2<T> (&x)[RA]) {
@@ -371,7 +445,7 @@ __device__ __forceinline__ void col_rest(const StageArgs &a, int blk, V2<T> (&x)
   const int sl = tid % C;
   const int t = tid / C;
   const int64_t u0 = static_cast<int64_t>(blk) * C;
-  const ColUnit un = col_unit<C>(a, blk, sl);
+  const ColUnit un = col_unit<C, MODE>(a, blk, sl);
   const bool active = un.active;
   const uint32_t bq = un.bq, i = un.i;
   const bool first = a.p == a.ncol;
@@ -380,6 +454,7 @@ __device__ __forceinline__ void col_rest(const StageArgs &a, int blk, V2<T> (&x)
   const uint32_t tcnt = static_cast<uint32_t>(a.tcnt);
   const uint32_t kmul = kt * static_cast<uint32_t>(a.twp_mult);
   const T scale = static_cast<T>(a.scale);
+  const uint32_t j0 = (static_cast<uint32_t>(u0) - bq * tcnt) / 2;  // first pair of a real tile
 
   // Bluestein chains: the last passes write conj(X bhat) (forward chain) or
   // conj(X) chirp for e < n = nlog (inverse chain)
@@ -391,6 +466,25 @@ __device__ __forceinline__ void col_rest(const StageArgs &a, int blk, V2<T> (&x)
 #pragma unroll
   for (int j = 0; j < RA; ++j) x[j].y *= cs;
   constexpr bool kExact = RA >= 32 || MODE == kColBluestein;
+  if constexpr (MODE == kColRealPre) {
+    // x[q] = X_m -> conj Z'_m, Z'_m = (X_m + conj X_{h-m}) + i conj(w_n^m) (X_m - conj X_{h-m})
+    // (conjugated: the inverse runs as a forward transform); Im of X_0 and X_h dropped
+    const V2<T> wb = real_twiddle<T>(a, i, tcnt, t);
+    const bool dc = i == 0 && t == 0;
+    V2<T> xn{0, 0};  // X_h, which no unit reads
+    if (dc) {
+      xn.x = ldt(gc<T>(a.in) + static_cast<int64_t>(bq) * a.bs_in, tcnt * static_cast<uint32_t>(R)).x;
+      x[0].y = T(0);
+    }
+    real_partner<T, C, RA, RB>(i, tcnt, t, sl, x, [&](auto Q, V2<T> xk, V2<T> xh, bool own) __attribute__((always_inline)) {
+      constexpr int q = decltype(Q)::value;
+      if (q == 0 && own) xh = xn;
+      const V2<T> c = cconj(xh);
+      const V2<T> u = twiddle_ct<q, 2 * RA>(cmul(wb, cconj(csub(xk, c))));  // conj(conj(w) (X_m - c))
+      return cconj(cadd(cadd(xk, c), cmul_pi(cconj(u))));
+    });
+    __syncthreads();  // its reads are done
+  }
   if (!first) col_twiddle<T, RA, RB, kExact>(a, kmul, t, x);
   V2<T> y[NM][RB];
   const bool bs = a.block_store != 0;
@@ -400,8 +494,9 @@ __device__ __forceinline__ void col_rest(const StageArgs &a, int blk, V2<T> (&x)
     if (bs) {
       // unit u0 + rsl owns outputs (u0 + rsl) R + e', e' = rk1 + RA k2
       if (u0 + rsl < a.units) {
-        GlbC<T> *dst = gc<T>(a.out) + u0 * R;
-        const uint32_t o0 = static_cast<uint32_t>(rsl * R + rk1);
+        GlbC<T> *dst = gc<T>(a.out) + (MODE == kColRealPre ? static_cast<int64_t>(bq) * a.bs_out : u0 * R);
+        const uint32_t us = MODE == kColRealPre ? pair_unit<C>(j0, tcnt, rsl) : static_cast<uint32_t>(rsl);
+        const uint32_t o0 = us * static_cast<uint32_t>(R) + static_cast<uint32_t>(rk1);
 #pragma unroll
         for (int q = 0; q < RB; ++q) {
           V2<T> v = y[0][q];
@@ -415,6 +510,31 @@ __device__ __forceinline__ void col_rest(const StageArgs &a, int blk, V2<T> (&x)
       }
       return;
     }
+  }
+
+  if constexpr (MODE == kColRealPost) {
+    // outputs e = t + RB q (q = m + NM k2) of the chain, Z_m, m = i + e p:
+    // X_m = E + w_n^m O, E = (Z_m + conj Z_{h-m}) / 2, O = -i (Z_m - conj Z_{h-m}) / 2
+    const uint32_t np = static_cast<uint32_t>(a.p);
+    const V2<T> wb = real_twiddle<T>(a, i, np, t);
+    V2<T> v[RA];
+#pragma unroll
+    for (int q = 0; q < RA; ++q) v[q] = y[q % NM][q / NM];
+    const V2<T> z0 = v[0];
+    const T half = T(0.5);
+    real_partner<T, C, RA, RB>(i, np, t, sl, v, [&](auto Q, V2<T> zk, V2<T> zh, bool) __attribute__((always_inline)) {
+      constexpr int q = decltype(Q)::value;
+      const V2<T> zc = cconj(zh);
+      const V2<T> ev{(zk.x + zc.x) * half, (zk.y + zc.y) * half};
+      const V2<T> od = cmul_mi(V2<T>{(zk.x - zc.x) * half, (zk.y - zc.y) * half});
+      return cadd(ev, twiddle_ct<q, 2 * RA>(cmul(wb, od)));
+    });
+    GlbC<T> *dst = gc<T>(a.out) + static_cast<int64_t>(bq) * a.bs_out;
+    const uint32_t o0 = i + static_cast<uint32_t>(t) * np;
+#pragma unroll
+    for (int q = 0; q < RA; ++q) stt(dst, o0 + static_cast<uint32_t>(RB * q) * np, v[q]);
+    if (i == 0 && t == 0) stt(dst, np * static_cast<uint32_t>(R), V2<T>{z0.x - z0.y, T(0)});
+    return;
   }
 
   auto finish = [&](V2<T> v) __attribute__((always_inline)) {
@@ -433,7 +553,8 @@ __device__ __forceinline__ void col_rest(const StageArgs &a, int blk, V2<T> (&x)
     // row pitch = 4 (mod 32) entries: the 16 slots of a wavefront's store land
     // on distinct bank octets
     constexpr int LSB = (BL + BL / 32 + 28) / 32 * 32 + 4;
-    GlbC<T> *dst = gc<T>(a.out) + u0 * R;
+    // (a real tile's units are contiguous rows of their own)
+    GlbC<T> *dst = gc<T>(a.out) + (MODE == kColRealPre ? static_cast<int64_t>(bq) * a.bs_out : u0 * R);
     const int64_t total = a.units * static_cast<int64_t>(R);
 #pragma unroll
     for (int d = 0; d < NCH; ++d) {
@@ -454,8 +575,9 @@ __device__ __forceinline__ void col_rest(const StageArgs &a, int blk, V2<T> (&x)
         const int f = tid + r * NT;
         if (f < C * BL) {
           const int s2 = f / BL, e2 = f - s2 * BL;
-          const int64_t g = static_cast<int64_t>(s2) * R + d * BL + e2;
-          if (u0 * R + g < total) stg(dst + g, finish(ldc(lds + s2 * LSB + e2 + (e2 >> 5))));
+          const int64_t us = MODE == kColRealPre ? pair_unit<C>(j0, tcnt, s2) : s2;
+          const int64_t g = us * R + d * BL + e2;
+          if (MODE == kColRealPre || u0 * R + g < total) stg(dst + g, finish(ldc(lds + s2 * LSB + e2 + (e2 >> 5))));
         }
       }
     }
@@ -576,7 +698,7 @@ __device__ __forceinline__ void col_conv_body(const StageArgs &a, int blk) {
   const int sl = tid % C;
   const int t = tid / C;
   const int64_t u0 = static_cast<int64_t>(blk) * C;
-  const ColUnit un = col_unit<C>(a, blk, sl);
+  const ColUnit un = col_unit<C, kColPlain>(a, blk, sl);
   const uint32_t i = un.i, p = static_cast<uint32_t>(a.p);
   const uint32_t k = i - fdiv(i, a.fd_p) * p;
   V2<T> x[RA], y[1][RA];

@@ -112,6 +112,7 @@ size_t Step::pack_args(void *src, void *dst, unsigned char *buf, void *aux) cons
     case Pass: return put(pa);
     case Leaf: return put(la);
     case Stage:
+    case ColReal:
     case Col: return put(sa);
     case Mfma: return put(ma);
     case BluesteinLds: {
@@ -165,6 +166,15 @@ Step Step::rebatched(int64_t batch, int64_t built) const {
       if (!col_tiles_fit(sa.tcnt, sa.p, col_kernel_radix(leaf_id), per, sa.bs_in, sa.bs_out, s.sa.units / sa.tcnt, ebytes))
         throw std::logic_error("re-batched pass whose tiles span 4 GiB");
       s.sa.nblocks = static_cast<int32_t>(blocks(s.sa.units, per));
+      s.shape.grid = dim3(static_cast<unsigned>(s.sa.nblocks));
+      break;
+    }
+    case ColReal: {
+      int per = 1, thr = 0, ebytes = 0;
+      size_t lds = 0;
+      col_real_kernel_shape(leaf_id, per, thr, lds, ebytes);  // whole tiles of one sequence
+      s.sa.units = scale(sa.units);
+      s.sa.nblocks = static_cast<int32_t>(s.sa.units / per);
       s.shape.grid = dim3(static_cast<unsigned>(s.sa.nblocks));
       break;
     }
@@ -291,6 +301,7 @@ void Executable::resolve_kernels() {
                  : s.leaf_mode == 1 ? col_pair_kernel(s.leaf_id)
                                     : col_kernel(s.leaf_id, s.leaf_mode == 3);
         break;
+      case Step::ColReal: s.func = col_real_kernel(s.leaf_id, s.leaf_mode == 1); break;
       case Step::Mfma: s.func = mfma_kernel(s.compute, s.leaf_id); break;
       case Step::BluesteinLds: s.func = bluestein_lds_kernel(s.leaf_id, s.leaf_mode); break;
       case Step::BluesteinCombine: s.func = bluestein_combine_kernel(s.dbl, s.split); break;
@@ -1082,10 +1093,80 @@ void Builder::emit_multipass(const Core &c, const SeqSet &s, int src, int dst, c
     a.nlog = nl ? nl : n;
     if ((a.src_mode & kSrcChirpFlag) || (a.dst_mode & kDstChirpFlag)) a.chirp = chirp(a.nlog);
     // the pointwise pass of a Bluestein chain gets its table from emit_bluestein
-    if (!try_stage(a, c.pass_radices[j], 0, st_src, st_dst, s, n, static_cast<int>(j), static_cast<int>(k)))
+    const bool fused = (real_fuse_ == 1 && j + 1 == k) || (real_fuse_ == 2 && j == 0);
+    if (fused)
+      emit_col_real(a, st_src, st_dst, s, real_fuse_ == 1, static_cast<int>(j), static_cast<int>(k));
+    else if (!try_stage(a, c.pass_radices[j], 0, st_src, st_dst, s, n, static_cast<int>(j), static_cast<int>(k)))
       emit_pass_step(a, st_src, st_dst, s, n, static_cast<int>(j), static_cast<int>(k));
     p *= R;
   }
+}
+
+// Whether the split-spectrum pass of a real transform with this n/2-point chain
+// runs in its last (fwd) or first pass: a register-resident instance of that
+// super-radix whose tile divides a sequence's units, contiguous rows.
+bool Builder::can_fuse_real(const Core &c, const SeqSet &s, bool fwd) {
+  if (c.kind != CoreKind::MultiPass || opt_.generic_kernels || opt_.stage_form == 2 || opt_.forced_units != 0 ||
+      s.col_fast || s.ncol != 1 || s.gi.es != 1 || s.go.es != 1 || (fwd ? s.gi.bs : s.go.bs) % 2 != 0)
+    return false;
+  const int64_t r = fwd ? c.passes.back() : c.passes.front(), tcnt = c.n / r;
+  const int id = col_real_kernel_id(r, dbl(), tcnt, s.nbatch * tcnt);
+  return id >= 0 && s.nbatch * tcnt < (int64_t{1} << 31) && (c.n + 1) * eb() < (int64_t{1} << 32);
+}
+
+void Builder::emit_col_real(const PassArgs &a, int src, int dst, const SeqSet &s, bool post, int pass, int npasses) {
+  const int id = col_real_kernel_id(a.R, dbl(), a.tcnt, a.units);
+  int units = 0, threads = 0, ebytes = 0;
+  size_t lds = 0;
+  col_real_kernel_shape(id, units, threads, lds, ebytes);
+  const int64_t h = a.nseq;
+  const TwoLevel tl = two_level(2 * h);
+  Step st;
+  st.kind = Step::ColReal;
+  st.dbl = dbl();
+  st.src = src;
+  st.dst = dst;
+  st.leaf_id = id;
+  st.leaf_mode = post ? 1 : 2;
+  StageArgs &g = st.sa;
+  g.bs_in = a.gi.bs;
+  g.bs_out = a.go.bs;
+  g.tcnt = a.tcnt;
+  g.p = a.p;
+  g.twp_mult = a.twp_mult;
+  g.tw_bits = a.tw_bits;
+  g.fd_tcnt = make_fastdiv(static_cast<uint32_t>(a.tcnt));
+  g.fd_p = make_fastdiv(static_cast<uint32_t>(a.p));
+  g.ncol = 1;
+  g.fd_ncol = make_fastdiv(1);
+  g.tw_small = a.tw_small;
+  g.tw_lo = a.tw_lo;
+  g.tw_hi = a.tw_hi;
+  g.conj_in = 0;
+  g.conj_out = a.conj_out;
+  g.scale = a.scale;
+  g.units = a.units;
+  g.block_store = post ? 0 : 1;
+  g.src_mode = kSrcComplex;
+  g.dst_mode = kDstComplex;
+  g.nlog = h;
+  g.chirp = nullptr;
+  g.bhat = nullptr;
+  g.dc_nyq_pair = 0;
+  g.stream = 0;
+  g.tw_rlo = tl.lo;
+  g.tw_rhi = tl.hi;
+  g.tw_rbits = tl.bits;
+  g.nblocks = static_cast<int32_t>(a.units / units);
+  g.xcd_remap = opt_.xcd_remap;
+  st.ept = 0;
+  st.shape = LaunchShape{dim3(static_cast<unsigned>(g.nblocks)), dim3(static_cast<unsigned>(threads)), lds};
+  st.bytes_moved = s.nbatch * (2 * h + 1) * eb();
+  std::ostringstream lab;
+  lab << "k_col_real<" << (dbl() ? "fp64" : "fp32") << "," << col_real_targs(id, post) << "> pass " << pass << "/"
+      << npasses << " R=" << a.R << " p=" << a.p << " tcnt=" << a.tcnt << " n=" << 2 * h;
+  st.label = lab.str();
+  ex_.steps.push_back(st);
 }
 
 void Builder::emit_rader(const Core &c, const SeqSet &s, int src, int dst, const Modes &m) {
@@ -1711,6 +1792,16 @@ void Builder::emit_plan1d(const Plan1D &pl, const SeqSet &s, int src, int dst, b
   // EvenMulti: n/2-point core (multi-pass chain, Rader or Bluestein) plus a split-spectrum pass
   const Geometry gws{1, h, h * s.ncol};
   const size_t wbytes = static_cast<size_t>(s.nbatch * s.ncol * h) * eb();
+  if (SeqSet sc = s; can_fuse_real(pl.core, s, pl.real_fwd)) {
+    Modes m;
+    (pl.real_fwd ? sc.gi : sc.go) =
+        pl.real_fwd ? Geometry{1, s.gi.cs / 2, s.gi.bs / 2} : Geometry{1, s.go.cs / 2, s.go.bs / 2};
+    m.conj_out = !pl.real_fwd;
+    real_fuse_ = pl.real_fwd ? 1 : 2;
+    emit_multipass(pl.core, sc, src, dst, m, m, {});
+    real_fuse_ = 0;
+    return;
+  }
   const TwoLevel tw = two_level(n);
   if (pl.real_fwd) {
     const int W = pick_ws({src, dst}, wbytes);

@@ -53,7 +53,8 @@ struct Step {
     RealPost,
     RealPre,
     Mfma,
-    Col
+    Col,
+    ColReal  // Col with the split-spectrum pass of a real transform (leaf_mode: 1 post, 2 pre)
   } kind = Pass;
   bool dbl = false;
   int ept = 16;
@@ -182,6 +183,7 @@ class Builder {
   std::vector<std::shared_ptr<DevBuf>> temps_;
   std::vector<std::unique_ptr<Executable>> temp_execs_;
   int pair_ = 0, pair_steps_ = 0;
+  int real_fuse_ = 0;  // split-spectrum pass in the chain emitted next: 1 in its last pass, 2 in its first
 
   bool dbl() const { return prec_ == Prec::F64; }
   int eb() const { return elem_bytes(prec_); }
@@ -214,6 +216,8 @@ class Builder {
   void emit_bluestein(const Core &c, const SeqSet &s, int src, int dst, const Modes &m);
   bool conv_ends_in_registers(int64_t r0, int64_t M, const SeqSet &s);
   void emit_bluestein_split(const Core &c, const SeqSet &s, int src, int dst, const Modes &m, int split);
+  bool can_fuse_real(const Core &c, const SeqSet &s, bool fwd);
+  void emit_col_real(const PassArgs &a, int src, int dst, const SeqSet &s, bool post, int pass, int npasses);
   bool try_leaf_split(const Core &c, const SeqSet &s, int src, int dst, const Modes &m);
   bool try_leaf_split_real(const Plan1D &pl, const SeqSet &s, int src, int dst);
   void emit_leaf_split(int id, int mode, int64_t n, int64_t nseq, int64_t idist, int64_t odist, int src, int dst,

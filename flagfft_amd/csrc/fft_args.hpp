@@ -191,6 +191,10 @@ struct StageArgs {
   //      whose inverse transform is Re IFFT A + i Re IFFT B
   int32_t dc_nyq_pair;
   int32_t stream;  // StreamHint bits (register-resident passes)
+  // passes fused with the split-spectrum pass of a real transform of n = 2 nseq
+  // points: w_n^k = tw_rhi[k >> tw_rbits] tw_rlo[k & (2^tw_rbits - 1)]
+  int32_t tw_rbits;
+  const void *tw_rlo, *tw_rhi;
 };
 
 // Bluestein with the whole convolution in LDS (one sequence per workgroup).

@@ -83,6 +83,12 @@ int col_queue_variant(int id);
 int col_conv_kernel_id(int64_t r, bool dbl, int64_t total_units);
 const void *col_conv_kernel(int id);
 std::string col_conv_targs(int id);
+// Passes fused with the split-spectrum pass of an even-length real transform:
+// the instance for tcnt units per sequence, which its tile divides (-1: none).
+int col_real_kernel_id(int64_t r, bool dbl, int64_t tcnt, int64_t total_units);
+void col_real_kernel_shape(int id, int &units, int &threads, size_t &lds_bytes, int &elem_bytes);
+const void *col_real_kernel(int id, bool post);
+std::string col_real_targs(int id, bool post);
 // Template arguments after the element type, as the kernel symbol lists them.
 std::string col_kernel_targs(int id, int mode);  // mode: ColMode
 
