@@ -845,7 +845,9 @@ Builder::TwoLevel Builder::two_level(int64_t n) {
 
 bool Builder::try_stage(const PassArgs &a, const std::vector<int> &radices, int mode, int src, int dst,
                         const SeqSet &s, int64_t n, int pass, int npasses) {
-  const int sid = opt_.generic_kernels ? -1 : stage_kernel_id(radices, dbl(), opt_.forced_units);
+  const int sid = opt_.generic_kernels        ? -1
+                  : opt_.forced_units != 0 ? stage_kernel_id(radices, dbl(), opt_.forced_units)
+                                           : stage_kernel_id_for(radices, dbl(), a.units);
   // register-resident two-stage pass (plain complex passes, and Bluestein
   // chain ends: chirp source, pointwise and chirp sinks)
   const bool col_allowed = mode == 0 && opt_.stage_form != 2 && (!opt_.generic_kernels || opt_.queue_form) &&

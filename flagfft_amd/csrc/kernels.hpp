@@ -45,6 +45,9 @@ int stage_kernel_id(const std::vector<int> &radices);
 std::vector<int64_t> stage_kernel_radices();  // the super-radices of all instances
 // The instance with `units` per workgroup (0: the default one), -1 if none.
 int stage_kernel_id(const std::vector<int> &radices, bool dbl, int units);
+// The instance for a launch of total_units: a narrower one while the default one's
+// tiles give fewer than one workgroup per CU.
+int stage_kernel_id_for(const std::vector<int> &radices, bool dbl, int64_t total_units);
 void stage_kernel_shape(int id, bool dbl, int &units_per_group, int &ept);
 const void *stage_kernel(bool dbl, int id, int mode);  // mode: 0 chain pass, 1 Bluestein convolution
 // False for the instances that beat only the run-time-radix pass (5- and

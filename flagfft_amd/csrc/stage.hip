@@ -5,6 +5,8 @@
 // restated as Stockham passes with fused twiddles).
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
+
 #include "codelets.hpp"
 #include "dev_common.hpp"
 #include "fft_args.hpp"
@@ -94,13 +96,22 @@ __global__ __launch_bounds__(kMaxBlockThreads) void k_stage(const StageArgs a) {
     });
   };
 
-  auto load_global = [&](int e) __attribute__((always_inline)) {
+  // Straight-line loads (idle slots read unit 0): a load under a mask or a branch
+  // waits for the one before it (10^6 x 8: 73 + 61 -> 44 + 43 us, 125-point passes of
+  // 500000 x 4 20 -> 15).
+  const T cs = a.conj_in ? T(-1) : T(1);
+  auto load_plain = [&](int e) __attribute__((always_inline)) {
+    V2<T> v = ldg(src + (static_cast<int64_t>(i) + e * tcnt));
+    v.y *= cs;
+    return v;
+  };
+  auto load_chirp = [&](int e) __attribute__((always_inline)) {
     const int64_t elog = static_cast<int64_t>(i) + e * tcnt;
     V2<T> v{0, 0};
-    if (active && !(chirp_in && elog >= a.nlog)) {
+    if (active && elog < a.nlog) {
       v = ldg(src + elog);
-      if (a.conj_in) v.y = -v.y;
-      if (chirp_in) v = cmul(v, ldg(chirp + elog));
+      v.y *= cs;
+      v = cmul(v, ldg(chirp + elog));
     }
     return v;
   };
@@ -109,7 +120,7 @@ __global__ __launch_bounds__(kMaxBlockThreads) void k_stage(const StageArgs a) {
   bool block_store = a.block_store != 0;
   if constexpr (Mode == kStageConvolution) {
     block_store = true;
-    run_stages<T, E, TPU, RS, false, 5, true>(buf, t, twr, tws, true, load_global, to_lds, pre0);
+    run_stages<T, E, TPU, RS, false, 5, true>(buf, t, twr, tws, true, load_plain, to_lds, pre0);
     __syncthreads();
     const GlbC<T> *bhat = gc<T>(a.bhat);
     run_stages<T, E, TPU, RS, true, 5, true>(
@@ -118,18 +129,25 @@ __global__ __launch_bounds__(kMaxBlockThreads) void k_stage(const StageArgs a) {
           return cconj(cmul(ldc(buf + lpad(e)), ldg(bhat + (i + static_cast<int64_t>(e) * a.p))));
         },
         to_lds);
-  } else if (block_store) {
-    run_stages<T, E, TPU, RS, false, 5, true>(buf, t, twr, tws, true, load_global, to_lds, pre0);
   } else {
-    run_stages<T, E, TPU, RS, false, 5, true>(
-        buf, t, twr, tws, false, load_global,
-        [&](int idx, V2<T> v) __attribute__((always_inline)) {
-          if (!active) return;
-          const int64_t oidx = (i - k) * static_cast<int64_t>(R) + k + static_cast<int64_t>(idx) * a.p;
-          dst_elem<T>(a.out, static_cast<int64_t>(bq) * a.bs_out, 1, a.dst_mode, a.nlog, a.chirp, a.bhat,
-                      a.conj_out, scale, oidx, v);
-        },
-        pre0);
+    auto run = [&](auto load) __attribute__((always_inline)) {
+      if (block_store)
+        run_stages<T, E, TPU, RS, false, 5, true>(buf, t, twr, tws, true, load, to_lds, pre0);
+      else
+        run_stages<T, E, TPU, RS, false, 5, true>(
+            buf, t, twr, tws, false, load,
+            [&](int idx, V2<T> v) __attribute__((always_inline)) {
+              if (!active) return;
+              const int64_t oidx = (i - k) * static_cast<int64_t>(R) + k + static_cast<int64_t>(idx) * a.p;
+              dst_elem<T>(a.out, static_cast<int64_t>(bq) * a.bs_out, 1, a.dst_mode, a.nlog, a.chirp, a.bhat,
+                          a.conj_out, scale, oidx, v);
+            },
+            pre0);
+    };
+    if (chirp_in)
+      run(load_chirp);
+    else
+      run(load_plain);
   }
   if (block_store) {
     // the workgroup's C units own one contiguous block of C * R output elements
@@ -200,8 +218,8 @@ const StageEntry kStageTable[] = {
     FLAGFFT_STAGE2(16, 16, 8, 16, 15, 9),       // 135
     FLAGFFT_STAGE3(8, 16, 4, 16, 9, 9, 9),      // 729
     // 5- and 10-smooth passes (10^k, 5^k lengths): the run-time-radix pass
-    // reads them at 0.4-0.9 TB/s, these at 0.9-1.9 (MI355X, 8-32 MB
-    // transforms), well below the power-of-two passes
+    // reads them at 0.4-0.9 TB/s, these at 0.9-2.9 (8-64 MB transforms),
+    // below the power-of-two passes
     FLAGFFT_STAGE2_SLOW(64, 16, 32, 16, 5, 5),       // 25
     FLAGFFT_STAGE2_SLOW(32, 16, 16, 16, 10, 10),     // 100
     FLAGFFT_STAGE3_SLOW(32, 16, 16, 16, 5, 5, 5),    // 125
@@ -214,6 +232,14 @@ const StageEntry kStageTable[] = {
     FLAGFFT_STAGE3(32, 32, 16, 16, 16, 16, 2),  // 512
     FLAGFFT_STAGE3(16, 32, 8, 16, 16, 16, 4),   // 1024
     FLAGFFT_STAGE3(8, 32, 4, 32, 16, 16, 8),    // 2048
+    // narrow tiles for launches that leave CUs idle otherwise, one butterfly of the
+    // largest radix per thread (a launch of 32-63 workgroups is latency: 1000 x 1000
+    // columns 30.4 -> 10.4 us, 10^6 x 1 57 -> 18, 729 x 729 columns 20.6 -> 8.8,
+    // 100 x 100 columns 14.3 -> 6.4)
+    FLAGFFT_STAGE3(4, 9, 4, 9, 9, 9, 9),           // 729
+    FLAGFFT_STAGE2_SLOW(8, 10, 8, 10, 10, 10),     // 100
+    FLAGFFT_STAGE3_SLOW(8, 5, 8, 5, 5, 5, 5),      // 125
+    FLAGFFT_STAGE3_SLOW(4, 10, 4, 10, 10, 10, 10), // 1000
 };
 
 }  // namespace
@@ -231,6 +257,19 @@ int stage_kernel_id(const std::vector<int> &radices, bool dbl, int units) {
     if (first < 0) first = i;
   }
   return units > 0 ? -1 : first;
+}
+
+int stage_kernel_id_for(const std::vector<int> &radices, bool dbl, int64_t total_units) {
+  const int n = static_cast<int>(sizeof(kStageTable) / sizeof(kStageTable[0]));
+  int best = stage_kernel_id(radices, dbl, 0);
+  if (best < 0) return best;
+  for (int i = best + 1; i < n; ++i) {
+    const StageEntry &e = kStageTable[i], &b = kStageTable[best];
+    if (e.nrad != b.nrad || !std::equal(e.rad, e.rad + 3, b.rad)) continue;
+    const int c = dbl ? e.c64 : e.c32, bc = dbl ? b.c64 : b.c32;
+    if (c < bc && total_units < int64_t{256} * bc) best = i;
+  }
+  return best;
 }
 
 int stage_kernel_id(const std::vector<int> &radices) { return stage_kernel_id(radices, false, 0); }
