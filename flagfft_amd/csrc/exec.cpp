@@ -1381,14 +1381,17 @@ void Builder::emit_bluestein(const Core &c, const SeqSet &s, int src, int dst, c
       split = 4;
     } else if (opt_.forced_units < 1 || opt_.forced_units > 5) {
       // measured on MI355X: a whole convolution per workgroup stays ahead
-      // until fewer than 1/8 of the CUs have a sequence; the two-halves form
+      // while more than 1/4 of the CUs have a sequence; below, splits in 4
+      // (FP32, 10007 x 33 / 48 / 64: 22.5 / 22.6 / 23.3 -> 16.8 / 19.7 / 22.1 us,
+      // 5003 x 64: 20.6 -> 17.1) or, until 1/8, in 2 (FP64, 5003 x 33 / 64:
+      // 19.6 / 20.1 -> 16.5 / 19.6; in 4 20.9 at 64).  The two-halves form
       // (two convolutions in a row per workgroup) splits in 2 below 1/2
       // (in 4 below 1/8: the combine pass reads P blocks, so P = 2 costs
       // less device time when the GPU is shared)
       const int ncu = cu_count();
-      if (nseqs_all * 8 <= ncu)
+      if (nseqs_all * 8 <= ncu || (!dbl() && !c.lds_halves && nseqs_all * 4 <= ncu))
         split = 4;
-      else if (c.lds_halves && nseqs_all * 2 <= ncu)
+      else if (c.lds_halves ? nseqs_all * 2 <= ncu : nseqs_all * 4 <= ncu)
         split = 2;
     }
     if (split > 0 && bluestein_split_kernel_id(M, dbl(), split) < 0) split = split == 4 ? 2 : 0;
