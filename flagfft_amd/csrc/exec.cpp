@@ -11,9 +11,9 @@ namespace flagfft {
 namespace {
 // Inputs from half the Infinity Cache on are read with non-temporal loads: input
 // and workspace (or output) no longer fit it together.  4096^2 C2C 111 -> 103 us,
-// 256^3 C2C 143 -> 130, 2^24 C2C 143 -> 133; inputs of 64 MiB would lose (256^3
-// R2C 73 -> 79, 2048 x 4096 C2C 53.5 -> 56.5: the last pass over them often finds
-// them cached).
+// 256^3 C2C 143 -> 130, 2^24 C2C 143 -> 133, 2^20 x 32 260 -> 199; inputs of 64 MiB
+// would lose (256^3 R2C 73 -> 79, 2048 x 4096 C2C 53.5 -> 56.5: the last pass over
+// them often finds them cached).
 constexpr int64_t kStreamInBytes = int64_t{128} << 20;
 // Outputs of single-pass rows up to this size are written with non-temporal
 // stores, which leave less to write back at the launch's end.  They do not stay in
@@ -232,15 +232,20 @@ void Step::set_stream_hints() {
       // as for Col below, whole lines: the last stage stores runs of tpu
       // elements, N / radix apart (64 x 65536, 32-byte runs: 13.6 -> 30.3 us
       // with the hint; 1000 x 16000, 800 bytes apart: 53.5 -> 56.4).  R2C rows
-      // (N + 1 bins) are never whole lines and gain all the same
+      // (N + 1 bins) are never whole lines and gain all the same.  C2R rows'
+      // loads, for the same reason, do not (1024 points x 76800 116 -> 120 us)
       const int64_t eb = dbl ? 16 : 8, tpu = shape.block.x / static_cast<unsigned>(la.C);
+      in = in && leaf_mode != kRowC2R && stream_row_loads(static_cast<int>(tpu), static_cast<int>(eb)) &&
+           la.idist * eb % 128 == 0 && leaf_kernel_first_stride(leaf_id) * eb % 128 == 0;
       out = out && output_bytes <= kStreamOutBytes && tpu * eb >= 128 &&
             (leaf_mode == kRowR2C || (la.odist * eb % 128 == 0 && leaf_kernel_last_stride(leaf_id) * eb % 128 == 0));
       la.stream = bits();
       break;
     }
     case RealPost:
-    case RealPre: ra.stream = bits(); break;
+      in = false;
+      ra.stream = bits();
+      break;
     case Col: {
       // whole 128-byte lines only: a tile's row segment under that, or across
       // a line's end, meets the rest of the line from another workgroup, which
@@ -262,10 +267,16 @@ void Step::set_stream_hints() {
 
 void Executable::mark_streams(int64_t in_bytes, int64_t out_bytes) {
   int readers = 0;
-  for (const Step &s : steps) readers += s.src == kBufIn ? 1 : 0;
+  bool post = false;  // a split-spectrum pass ends the rows' chain
+  for (const Step &s : steps) {
+    readers += s.src == kBufIn ? 1 : 0;
+    post = post || s.kind == Step::RealPost || (s.kind == Step::ColReal && s.leaf_mode == 1);
+  }
   for (size_t i = 0; i < steps.size(); ++i) {
     Step &s = steps[i];
-    s.input_bytes = s.src == kBufIn && readers == 1 ? in_bytes : 0;
+    // (not the first pass of an R2C chain: 2^20 x 65 320 -> 332 us with the hint,
+    // FP64 x 32 278 -> 295)
+    s.input_bytes = s.src == kBufIn && readers == 1 && !(s.kind == Step::Col && post) ? in_bytes : 0;
     s.output_bytes = s.dst == kBufOut ? out_bytes : 0;
     for (size_t j = i + 1; j < steps.size(); ++j)
       if (steps[j].src == kBufOut || steps[j].dst == kBufOut) s.output_bytes = 0;
@@ -450,8 +461,10 @@ std::string Executable::describe() const {
   o << "kernels=" << steps.size() << " workspaces=" << ws_bytes.size() << "\n";
   for (size_t i = 0; i < steps.size(); ++i) {
     const Step &s = steps[i];
+    const int hints = s.kind == Step::Leaf ? s.la.stream : s.kind == Step::Col ? s.sa.stream : s.ra.stream;
     o << "  [" << i << "] " << s.label << " " << buf_name(s.src) << "->" << buf_name(s.dst) << " grid=" << s.shape.grid.x
-      << " block=" << s.shape.block.x << " lds=" << s.shape.lds_bytes << "\n";
+      << " block=" << s.shape.block.x << " lds=" << s.shape.lds_bytes << ((hints & kStreamIn) ? " stream-in" : "")
+      << ((hints & kStreamOut) ? " stream-out" : "") << "\n";
   }
   return o.str();
 }

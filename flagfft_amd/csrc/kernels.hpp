@@ -36,6 +36,7 @@ LaunchShape real_pre_shape(const RealPassArgs &a);
 // Specialised single-pass kernels: id of the compiled radix sequence (-1 if none).
 int leaf_kernel_id(const std::vector<int> &radices);
 int leaf_kernel_ept(int id, bool dbl);
+int leaf_kernel_first_stride(int id);  // elements between the inputs of a first-stage butterfly
 int leaf_kernel_last_stride(int id);  // elements between the outputs of a last-stage butterfly
 const void *leaf_kernel(bool dbl, int id, int mode);  // mode: 0 complex, 1 R2C, 2 C2R
 

@@ -50,6 +50,7 @@ __global__ __launch_bounds__(kMaxBlockThreads) void k_leaf(const LeafArgs a) {
   const GlbC<T> *wn = gc<T>(a.aux);
   const GlbC<T> *tw = gc<T>(a.tw);
   V2<T> twr[RS::template pow_total<E>()];  // base twiddles of the inner stages
+  constexpr bool kHintLoads = stream_row_loads(TPU, sizeof(V2<T>));
   // split-spectrum passes: thread t handles k = t + i TPU, k <= N/2; every
   // table (and, for C2R, input) load of them is issued before any is used,
   // so their latencies overlap instead of one round trip per k
@@ -65,20 +66,14 @@ __global__ __launch_bounds__(kMaxBlockThreads) void k_leaf(const LeafArgs a) {
   if constexpr (Mode == kLeafC2R) {
     // fused pre-process into LDS (conjugated: the inverse runs as a forward transform)
     V2<T> xks[NK], xhs[NK];
-    auto load_bins = [&](auto ld) __attribute__((always_inline)) {
 #pragma unroll
-      for (int i = 0; i < NK; ++i) {
-        // (lanes past N / 2 read its bin; idle slots point at sequence 0.  A
-        // paired row carries X_N's real part in Im X_0: bin 0 stands for bin N)
-        const int k = min(t + i * TPU, N / 2);
-        xks[i] = ld(src + k);
-        xhs[i] = ld(src + (k == 0 && a.dc_nyq_pair ? 0 : N - k));
-      }
-    };
-    if (a.stream & kStreamIn)
-      load_bins([](const GlbC<T> *p) __attribute__((always_inline)) { return ldg_nt<T>(p); });
-    else
-      load_bins([](const GlbC<T> *p) __attribute__((always_inline)) { return ldg(p); });
+    for (int i = 0; i < NK; ++i) {
+      // (lanes past N / 2 read its bin; idle slots point at sequence 0.  A
+      // paired row carries X_N's real part in Im X_0: bin 0 stands for bin N)
+      const int k = min(t + i * TPU, N / 2);
+      xks[i] = ldg(src + k);
+      xhs[i] = ldg(src + (k == 0 && a.dc_nyq_pair ? 0 : N - k));
+    }
     prefetch_base_twiddles<T, E, TPU, RS>(twr, tw, t);
 #pragma unroll
     for (int i = 0; i < NK; ++i) {
@@ -124,7 +119,7 @@ __global__ __launch_bounds__(kMaxBlockThreads) void k_leaf(const LeafArgs a) {
           for (int j = 0; j < RR; ++j) x[m * RR + j] = ld(src + (b + j * NB));
         }
       };
-      if (a.stream & kStreamIn)
+      if (kHintLoads && (a.stream & kStreamIn))
         load_row([](const GlbC<T> *p) __attribute__((always_inline)) { return ldg_nt<T>(p); });
       else
         load_row([](const GlbC<T> *p) __attribute__((always_inline)) { return ldg(p); });
@@ -335,6 +330,13 @@ int leaf_kernel_last_stride(int id) {
   int q = 1;
   for (int j = 0; j + 1 < e.nrad; ++j) q *= e.rad[j];
   return q;
+}
+
+int leaf_kernel_first_stride(int id) {
+  const LeafEntry &e = kLeafTable[id];
+  int n = 1;
+  for (int j = 1; j < e.nrad; ++j) n *= e.rad[j];
+  return n;
 }
 
 const void *leaf_kernel(bool dbl, int id, int mode) { return kLeafTable[id].f[dbl ? 1 : 0][mode]; }
