@@ -21,6 +21,12 @@ constexpr int64_t kStreamInBytes = int64_t{128} << 20;
 // more: forward and inverse in a row, 4096 x 256 13.2 -> 12.1 us, x 1024 28.9 ->
 // 23.9, x 1536 42.5 -> 41.7, x 2048 49.4 -> 53.4, x 4096 90.5 -> 94.
 constexpr int64_t kStreamOutBytes = int64_t{32} << 20;
+// Half-spectrum rows from 2 MiB on: under it there is little to write back (R2C of
+// 2048 points, 1 / 4 / 12 MiB: 4.45 -> 4.70, 5.14 -> 5.02, 8.14 -> 7.51 us).  Rows of
+// under 48 threads, several to a wavefront's store, until 16 MiB (1024 points, 32
+// threads, 12 / 31 MiB: 8.7 -> 7.7, 12.8 -> 15.1; FP64 512 points, 16 threads, 12 / 24
+// MiB: 8.4 -> 7.4, 12.8 -> 14.2; 1536 points, 48 threads, 31 MiB: 18.2 -> 16.4).
+constexpr int64_t kStreamHalfRowBytes = int64_t{2} << 20, kStreamHalfRowShort = int64_t{16} << 20;
 }  // namespace
 
 void hip_check(hipError_t e, const char *what) {
@@ -231,14 +237,18 @@ void Step::set_stream_hints() {
     case Leaf: {
       // as for Col below, whole lines: the last stage stores runs of tpu
       // elements, N / radix apart (64 x 65536, 32-byte runs: 13.6 -> 30.3 us
-      // with the hint; 1000 x 16000, 800 bytes apart: 53.5 -> 56.4).  R2C rows
-      // (N + 1 bins) are never whole lines and gain all the same.  C2R rows'
-      // loads, for the same reason, do not (1024 points x 76800 116 -> 120 us)
+      // with the hint; 1000 x 16000, 800 bytes apart: 53.5 -> 56.4).  The N + 1
+      // bins of real rows are never whole lines: R2C stores gain all the same
+      // where runs are long, C2R loads do not (1024 points x 76800 116 -> 120 us)
       const int64_t eb = dbl ? 16 : 8, tpu = shape.block.x / static_cast<unsigned>(la.C);
       in = in && leaf_mode != kRowC2R && stream_row_loads(static_cast<int>(tpu), static_cast<int>(eb)) &&
            la.idist * eb % 128 == 0 && leaf_kernel_first_stride(leaf_id) * eb % 128 == 0;
-      out = out && output_bytes <= kStreamOutBytes && tpu * eb >= 128 &&
-            (leaf_mode == kRowR2C || (la.odist * eb % 128 == 0 && leaf_kernel_last_stride(leaf_id) * eb % 128 == 0));
+      out = out && output_bytes <= kStreamOutBytes &&
+            (leaf_mode == kRowR2C
+                 ? stream_half_rows(static_cast<int>(tpu), static_cast<int>(eb)) && output_bytes >= kStreamHalfRowBytes &&
+                       (tpu >= 48 || output_bytes <= kStreamHalfRowShort)
+                 : stream_row_stores(static_cast<int>(tpu), static_cast<int>(eb)) && la.odist * eb % 128 == 0 &&
+                       leaf_kernel_last_stride(leaf_id) * eb % 128 == 0);
       la.stream = bits();
       break;
     }

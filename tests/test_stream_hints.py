@@ -42,3 +42,19 @@ def test_loads(standin):
     for (t, n, b, want), steps in zip(LOADS, _launches(standin, [c[:3] for c in LOADS])):
         assert steps[0][1] == want, (t, n, b, steps)
         assert not any(s[1] for s in steps[1:]), (t, n, b, steps)
+
+
+# (type, n, batch, the output's stores are hinted): rows up to 32 MiB in whole lines;
+# half-spectrum rows from 2 MiB on in runs of 256 bytes, to 16 MiB or, with 48 threads
+# a row, 32
+STORES = [("C2C", 1024, 4096, True), ("C2C", 1024, 4097, False), ("C2C", 128, 4096, False), ("C2C", 256, 4096, True),
+          ("C2C", 1000, 2000, False), ("C2R", 4096, 2048, True), ("C2R", 4096, 2049, False),
+          ("R2C", 8, 300000, False), ("R2C", 32, 40000, False), ("R2C", 512, 8000, False), ("R2C", 1024, 4088, True),
+          ("R2C", 1024, 4090, False), ("D2Z", 256, 6000, False), ("D2Z", 512, 3000, True), ("D2Z", 512, 4100, False),
+          ("R2C", 1536, 2000, True), ("R2C", 2048, 256, True), ("R2C", 2048, 255, False),
+          ("R2C", 2048, 4091, True), ("R2C", 2048, 4093, False), ("D2Z", 1536, 1000, True)]
+
+
+def test_row_stores(standin):
+    for (t, n, b, want), steps in zip(STORES, _launches(standin, [c[:3] for c in STORES])):
+        assert len(steps) == 1 and steps[0][2] == want, (t, n, b, steps)
