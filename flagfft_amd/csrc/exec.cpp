@@ -27,6 +27,12 @@ constexpr int64_t kStreamOutBytes = int64_t{32} << 20;
 // threads, 12 / 31 MiB: 8.7 -> 7.7, 12.8 -> 15.1; FP64 512 points, 16 threads, 12 / 24
 // MiB: 8.4 -> 7.4, 12.8 -> 14.2; 1536 points, 48 threads, 31 MiB: 18.2 -> 16.4).
 constexpr int64_t kStreamHalfRowBytes = int64_t{2} << 20, kStreamHalfRowShort = int64_t{16} << 20;
+// Outputs of a split-spectrum pass of its own (k_real_post) from this size on:
+// smaller ones are faster left in the caches (R2C then C2R of 1002 points x 2092, 8
+// MiB, 84.5 us without and 85.6 with the hint, 752 x 8366, 24 MiB, 233.8 and 235.1),
+// larger ones written around them (1002 x 12557, 48 MiB, R2C 251 -> 222, there and
+// back the same; 200000 x 131 163 -> 146, 328 -> 316; 2^25 183 -> 174, 390 -> 375).
+constexpr int64_t kStreamPostBytes = int64_t{40} << 20;
 }  // namespace
 
 void hip_check(hipError_t e, const char *what) {
@@ -254,6 +260,7 @@ void Step::set_stream_hints() {
     }
     case RealPost:
       in = false;
+      out = out && output_bytes >= kStreamPostBytes;
       ra.stream = bits();
       break;
     case Col: {

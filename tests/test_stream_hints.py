@@ -58,3 +58,13 @@ STORES = [("C2C", 1024, 4096, True), ("C2C", 1024, 4097, False), ("C2C", 128, 40
 def test_row_stores(standin):
     for (t, n, b, want), steps in zip(STORES, _launches(standin, [c[:3] for c in STORES])):
         assert len(steps) == 1 and steps[0][2] == want, (t, n, b, steps)
+
+
+# the split-spectrum pass of its own: from 40 MiB on
+POST = [("R2C", 752, 419, False), ("R2C", 752, 13900, False), ("R2C", 752, 13920, True), ("D2Z", 1502, 3400, False),
+        ("D2Z", 1502, 3500, True), ("R2C", 1 << 25, 1, True)]
+
+
+def test_split_spectrum_pass(standin):
+    for (t, n, b, want), steps in zip(POST, _launches(standin, [c[:3] for c in POST])):
+        assert "k_real_post" in steps[-1][0] and steps[-1][2] == want, (t, n, b, steps)
