@@ -32,9 +32,10 @@ LOADS = [("C2C", 1024, 16384, True), ("C2C", 1024, 16383, False), ("C2C", 256, 1
          ("R2C", 64, 1 << 21, False), ("R2C", 256, 1 << 19, False), ("R2C", 512, 1 << 17, True), ("D2Z", 256, 1 << 17, True),
          # half-spectrum rows of N + 1 bins are never whole lines
          ("C2R", 128, 1 << 19, False), ("C2R", 4096, 1 << 14, False), ("Z2D", 64, 1 << 19, False),
-         # chains: the first pass, but of R2C (its output's write-back meets the next launch's loads)
-         ("C2C", 1 << 20, 16, True), ("C2C", 1 << 20, 15, False), ("Z2Z", 1 << 20, 16, True), ("R2C", 1 << 20, 64, False),
-         ("D2Z", 1 << 20, 32, False), ("R2C", 1 << 25, 2, False), ("C2R", 1 << 20, 64, False),
+         # chains: the first pass, of R2C up to 224 MiB
+         ("C2C", 1 << 20, 16, True), ("C2C", 1 << 20, 15, False), ("Z2Z", 1 << 20, 16, True), ("R2C", 1 << 20, 32, True),
+         ("R2C", 1 << 20, 31, False), ("R2C", 1 << 20, 55, True), ("R2C", 1 << 20, 56, False), ("D2Z", 1 << 20, 27, True),
+         ("D2Z", 1 << 20, 32, False), ("R2C", 1 << 25, 1, True), ("R2C", 1 << 25, 2, False), ("C2R", 1 << 20, 64, False),
          ("C2C", (4096, 4096), 1, True), ("R2C", (8192, 4096), 1, True), ("C2C", (256, 256, 256), 1, True)]
 
 
