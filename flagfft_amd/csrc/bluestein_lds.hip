@@ -344,7 +344,10 @@ __global__ __launch_bounds__(TPU) void k_bluestein_halves(const BluesteinLdsArgs
 // workgroup (q, h) convolves b_h against block h of bhat (digit-reversed over
 // [P, RS...]) and parks Z_h[e], e < min(ML, n); k_bluestein_combine applies
 // the radix-P last stage of the DIT transform.  tw = w_M^i, i < M.
-template <typename T, int TPU, int P, bool kFast, typename RS>
+// SRC: kSrcComplex / kSrcReal / kSrcHermitian of contiguous sequences, whose loads
+// are straight-line, or kSplitStrided for any source and stride.
+constexpr int kSplitStrided = 3;
+template <typename T, int TPU, int P, int SRC, typename RS>
 __device__ __forceinline__ void bluestein_split_body(const BluesteinLdsArgs &a) {
   constexpr int ML = RS::kN;
   constexpr int M = ML * P;
@@ -363,10 +366,11 @@ __device__ __forceinline__ void bluestein_split_body(const BluesteinLdsArgs &a) 
     slot = blockIdx.x;
   }
   const int h = static_cast<int>(slot % P);
-  const BlueIo<T, kFast> io(a, q);
+  const BlueIo<T, false> io(a, q);
   const int n = io.n;
   const GlbC<T> *tws = gc<T>(a.tw);
   GlbC<T> *park = gc<T>(a.park) + static_cast<int64_t>(slot) * ML;
+  const T cs = a.conj_in ? T(-1) : T(1);
   const GlbC<T> *cws = gc<T>(a.chirp_split) + static_cast<int64_t>(h) * n;
   conv_lds<T, TPU, false, P, RS::kR[0], RS::kR[0], RS>(
       lds_base<T>(), threadIdx.x, tws, gc<T>(a.bhat) + h * ML,
@@ -375,15 +379,31 @@ __device__ __forceinline__ void bluestein_split_body(const BluesteinLdsArgs &a) 
 #pragma unroll
         for (int j = 0; j < P / 2; ++j) {
           const int e2 = e + j * ML;
-          if (e2 < n) {
-            if constexpr (kFast) {
-              // x[e2] chirp[e2] w_M^(h e2) from one FP64-generated table
-              V2<T> xv = ldt(gc<T>(a.in) + io.ibase, static_cast<uint32_t>(e2));
-              if (a.conj_in) xv.y = -xv.y;
-              v = cadd(v, cmul(xv, ldt(cws, static_cast<uint32_t>(e2))));
+          const bool in = e2 < n;
+          if constexpr (SRC != kSplitStrided) {
+            // x[e2] chirp[e2] w_M^(h e2) from one FP64-generated table; straight-line
+            // loads, element 0 standing for those past the end (under a mask the
+            // table's value waited for the one before it: 10007 x 64 22.4 -> 17.5 us,
+            // and the step of six concurrent transforms with it 78 -> 74)
+            const uint32_t i2 = in ? static_cast<uint32_t>(e2) : 0u;
+            V2<T> xv;
+            if constexpr (SRC == kSrcReal) {
+              xv = V2<T>{(gr<T>(a.in) + io.ibase)[i2], T(0)};
+            } else if constexpr (SRC == kSrcHermitian) {
+              // bins past n / 2 mirror, Im of the bins that are their own dropped
+              const uint32_t nn = static_cast<uint32_t>(n);
+              const bool up = i2 > nn / 2;
+              xv = ldt(gc<T>(a.in) + io.ibase, up ? nn - i2 : i2);
+              xv.y = (i2 == 0 || 2 * i2 == nn) ? T(0) : up ? -xv.y : xv.y;
             } else {
-              v = cadd(v, cmul(io.in(e2), ldt(tws, static_cast<uint32_t>((h * e2) % M))));
+              xv = ldt(gc<T>(a.in) + io.ibase, i2);
             }
+            xv.y *= cs;
+            const V2<T> z = cmul(xv, ldt(cws, i2));
+            v.x += in ? z.x : T(0);
+            v.y += in ? z.y : T(0);
+          } else if (in) {
+            v = cadd(v, cmul(io.in(e2), ldt(tws, static_cast<uint32_t>((h * e2) % M))));
           }
         }
         return v;
@@ -393,13 +413,11 @@ __device__ __forceinline__ void bluestein_split_body(const BluesteinLdsArgs &a) 
       });
 }
 
-template <typename T, int TPU, int P, int... Rs>
+// (an instance per source: with all four in one the registers of the largest cost
+// complex sequences 7 %)
+template <typename T, int TPU, int P, int SRC, int... Rs>
 __global__ __launch_bounds__(TPU) void k_bluestein_split(const BluesteinLdsArgs a) {
-  using RS = RadixSeq<Rs...>;
-  if (a.gi.es == 1 && a.src_mode == kSrcComplex)
-    bluestein_split_body<T, TPU, P, true, RS>(a);
-  else
-    bluestein_split_body<T, TPU, P, false, RS>(a);
+  bluestein_split_body<T, TPU, P, SRC, RadixSeq<Rs...>>(a);
 }
 
 // W[e] = sum_h Z_h[e mod ML] w_M^(h e mod M), y[e] = conj(W[e]) chirp[e]
@@ -453,7 +471,7 @@ struct BluesteinLdsEntry {
   // variants: 0 Stockham stages, 1 Stockham with base twiddles prefetched at
   // kernel start, 2 in-place stages with table twiddles, 3 in-place stages
   // with binary-powered twiddles; entries without Stockham kernels hold
-  // their one kernel in every slot
+  // their one kernel in every slot, split ones a kernel per source (SRC)
   const void *f[4];
 };
 
@@ -476,10 +494,17 @@ struct BluesteinLdsEntry {
   FLAGFFT_BLDS_ONE(true, false, 0, TPU, (dev::k_bluestein_ip<double, TPU, false, R0, R1, R2, R3>), 4, R0, R1, R2, R3)
 #define FLAGFFT_BLDS_HALVES(T, DBL, TPU, R0, R1, R2, R3) \
   FLAGFFT_BLDS_ONE(DBL, true, 0, TPU, (dev::k_bluestein_halves<T, TPU, R0, R1, R2, R3>), 4, R0, R1, R2, R3)
-#define FLAGFFT_BLDS_SPLIT4(T, DBL, P, TPU, R0, R1, R2, R3) \
-  FLAGFFT_BLDS_ONE(DBL, false, P, TPU, (dev::k_bluestein_split<T, TPU, P, R0, R1, R2, R3>), 4, R0, R1, R2, R3)
-#define FLAGFFT_BLDS_SPLIT3(T, DBL, P, TPU, R0, R1, R2) \
-  FLAGFFT_BLDS_ONE(DBL, false, P, TPU, (dev::k_bluestein_split<T, TPU, P, R0, R1, R2>), 3, R0, R1, R2, 0)
+#define FLAGFFT_BLDS_SPLIT(T, DBL, P, TPU, NR, ...)                    \
+  {                                                                    \
+    DBL, false, P, NR, {__VA_ARGS__}, TPU, 0, {                       \
+      (const void *)dev::k_bluestein_split<T, TPU, P, 0, __VA_ARGS__>, \
+      (const void *)dev::k_bluestein_split<T, TPU, P, 1, __VA_ARGS__>, \
+      (const void *)dev::k_bluestein_split<T, TPU, P, 2, __VA_ARGS__>, \
+      (const void *)dev::k_bluestein_split<T, TPU, P, 3, __VA_ARGS__>  \
+    }                                                                  \
+  }
+#define FLAGFFT_BLDS_SPLIT4(T, DBL, P, TPU, R0, R1, R2, R3) FLAGFFT_BLDS_SPLIT(T, DBL, P, TPU, 4, R0, R1, R2, R3)
+#define FLAGFFT_BLDS_SPLIT3(T, DBL, P, TPU, R0, R1, R2) FLAGFFT_BLDS_SPLIT(T, DBL, P, TPU, 3, R0, R1, R2)
 
 // M in LDS: 16384 / 20160 complex FP32 and 8192 / 10080 complex FP64 (one
 // pad slot per 64 elements); the halves kernels reach twice those M, the

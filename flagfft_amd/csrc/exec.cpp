@@ -1316,7 +1316,7 @@ void Builder::emit_bluestein_split(const Core &c, const SeqSet &s, int src, int 
   st.aux = park;
   st.split = split;
   st.leaf_id = id;
-  st.leaf_mode = 0;
+  st.leaf_mode = s.gi.es == 1 ? m.src_mode & 3 : 3;  // the instance of this source (3: any, strided)
   BluesteinLdsArgs &a = st.ba;
   a.gi = s.gi;
   a.go = s.go;
@@ -1350,7 +1350,7 @@ void Builder::emit_bluestein_split(const Core &c, const SeqSet &s, int src, int 
   st.bytes_moved = nseqs * src_bytes(a.src_mode, n, n, eb());
   const char *pr = dbl() ? "fp64" : "fp32";
   std::ostringstream lab;
-  lab << "k_bluestein_split<" << pr << "," << tpu << "," << split << ">[";
+  lab << "k_bluestein_split<" << pr << "," << tpu << "," << split << "," << st.leaf_mode << ">[";
   for (size_t i = 0; i < rad.size(); ++i) lab << (i ? "x" : "") << rad[i];
   lab << "] n=" << n << " M=" << M << " transforms=" << nseqs;
   st.label = lab.str();
@@ -1416,9 +1416,13 @@ void Builder::emit_bluestein(const Core &c, const SeqSet &s, int src, int dst, c
     } else if (opt_.forced_units < 1 || opt_.forced_units > 5) {
       // measured on MI355X: a whole convolution per workgroup stays ahead
       // while more than 1/4 of the CUs have a sequence; below, splits in 4
-      // (FP32, 10007 x 33 / 48 / 64: 22.5 / 22.6 / 23.3 -> 16.8 / 19.7 / 22.1 us,
-      // 5003 x 64: 20.6 -> 17.1) or, until 1/8, in 2 (FP64, 5003 x 33 / 64:
-      // 19.6 / 20.1 -> 16.5 / 19.6; in 4 20.9 at 64).  The two-halves form
+      // (FP32, 10007 x 33 / 48 / 64: 22.5 / 22.9 / 23.9 -> 15.1 / 16.3 / 17.5 us,
+      // C2R x 64 26.8 -> 16.9) or, until 1/8, in 2 (FP64, 5003 x 33 / 64:
+      // 19.6 / 20.4 -> 15.8 / 17.5).  Beside other launches the split costs
+      // nothing for 10007 points (step of six families with 10007 x 64, three
+      // streams, 72.1-73.6 us whole and 71.3-72.4 split; with 10007 x 33 64.4 and
+      // 59.4) and something for 5003, whose whole form leaves half a CU's LDS (x 64:
+      // 55.6 whole, 59.0 split).  The two-halves form
       // (two convolutions in a row per workgroup) splits in 2 below 1/2
       // (in 4 below 1/8: the combine pass reads P blocks, so P = 2 costs
       // less device time when the GPU is shared)
