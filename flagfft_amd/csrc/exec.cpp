@@ -15,10 +15,12 @@ namespace {
 // would lose (256^3 R2C 73 -> 79, 2048 x 4096 C2C 53.5 -> 56.5: the last pass over
 // them often finds them cached).
 constexpr int64_t kStreamInBytes = int64_t{128} << 20;
-// First passes of R2C chains, whose input has as many bytes as the workspace and the
-// output each, gain below this size only: 2^20 x 32 / 40 / 50 / 64 (128 / 160 / 200 /
-// 256 MiB) 145 / 192 / 241 / 295 us without and 125 / 168 / 234 / 304 with the hint,
-// FP64 x 16 / 32 133 / 284 and 119 / 296, 2^25 x 1 192 and 175.
+// First passes of R2C chains and split-spectrum passes ahead of C2R ones, whose input
+// has as many bytes as the workspace and the output each, gain below this size only:
+// R2C of 2^20 x 32 / 40 / 50 / 64 (128 / 160 / 200 / 256 MiB) 145 / 192 / 241 / 295 us
+// without and 125 / 168 / 234 / 304 with the hint, FP64 x 16 / 32 133 / 284 and 119 /
+// 296, 2^25 x 1 192 and 175; C2R of 2^23 x 4 / 6 / 8 175 / 259 / 349 and 150 / 260 / 356,
+// 1502 points x 27924 / 34905 / 44679 616 / 778 / 994 and 536 / 727 / 995.
 constexpr int64_t kStreamRealInEnd = int64_t{224} << 20;
 // Outputs of single-pass rows up to this size are written with non-temporal
 // stores, which leave less to write back at the launch's end.  They do not stay in
@@ -263,6 +265,10 @@ void Step::set_stream_hints() {
       la.stream = bits();
       break;
     }
+    case RealPre:
+      out = false;
+      ra.stream = bits();
+      break;
     case RealPost:
       in = false;
       out = out && output_bytes >= kStreamPostBytes;
@@ -297,7 +303,7 @@ void Executable::mark_streams(int64_t in_bytes, int64_t out_bytes) {
   for (size_t i = 0; i < steps.size(); ++i) {
     Step &s = steps[i];
     s.input_bytes = s.src == kBufIn && readers == 1 ? in_bytes : 0;
-    if (s.kind == Step::Col && post && in_bytes >= kStreamRealInEnd) s.input_bytes = 0;
+    if (((s.kind == Step::Col && post) || s.kind == Step::RealPre) && in_bytes >= kStreamRealInEnd) s.input_bytes = 0;
     s.output_bytes = s.dst == kBufOut ? out_bytes : 0;
     for (size_t j = i + 1; j < steps.size(); ++j)
       if (steps[j].src == kBufOut || steps[j].dst == kBufOut) s.output_bytes = 0;

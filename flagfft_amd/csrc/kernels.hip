@@ -850,8 +850,8 @@ __device__ __forceinline__ void real_pre_body(const RealPassArgs &a, int blk, in
     const GlbC<T> *Xs = gc<T>(a.in) + b * a.gi.bs + c * a.gi.cs;
     GlbC<T> *Zo = gc<T>(a.out) + b * a.go.bs + c * a.go.cs;
     const GlbC<T> *pk = Xs + k * a.gi.es, *ph = Xs + (h - k) * a.gi.es;
-    V2<T> xk = ldg(pk);
-    V2<T> xh = ldg(ph);
+    V2<T> xk = (a.stream & kStreamIn) ? ldg_nt<T>(pk) : ldg(pk);
+    V2<T> xh = (a.stream & kStreamIn) ? ldg_nt<T>(ph) : ldg(ph);
     if (k == 0) {
       xk.y = T(0);
       xh.y = T(0);

@@ -36,6 +36,9 @@ LOADS = [("C2C", 1024, 16384, True), ("C2C", 1024, 16383, False), ("C2C", 256, 1
          ("C2C", 1 << 20, 16, True), ("C2C", 1 << 20, 15, False), ("Z2Z", 1 << 20, 16, True), ("R2C", 1 << 20, 32, True),
          ("R2C", 1 << 20, 31, False), ("R2C", 1 << 20, 55, True), ("R2C", 1 << 20, 56, False), ("D2Z", 1 << 20, 27, True),
          ("D2Z", 1 << 20, 32, False), ("R2C", 1 << 25, 1, True), ("R2C", 1 << 25, 2, False), ("C2R", 1 << 20, 64, False),
+         # the split-spectrum pass of its own ahead of a C2R chain, to 224 MiB as well
+         ("C2R", 1 << 24, 2, True), ("C2R", 1502, 27924, True), ("C2R", 1502, 22000, False), ("C2R", 1502, 39200, False),
+         ("Z2D", 1 << 23, 2, True), ("C2R", 1 << 24, 4, False),
          ("C2C", (4096, 4096), 1, True), ("R2C", (8192, 4096), 1, True), ("C2C", (256, 256, 256), 1, True)]
 
 
