@@ -222,7 +222,11 @@ int col_kernel_id_for(int64_t r, bool dbl, bool first, int64_t total_units, bool
   for (int id = 0; id < n; ++id) {
     const ColEntry &e = kColTable[id], &b = kColTable[best];
     if (e.r != r || e.dbl != dbl || (e.pref & 4) == 0) continue;
-    if (total_units < static_cast<int64_t>(kColGroups) * b.c && e.c < b.c) best = id;
+    // (FP64: while the narrower workgroups are one per CU at most.  256-point passes
+    // of 65536 x 8 / 10 / 12 in 128 / 160 / 192 workgroups of 16 14.3 / 15.7 / 16.5 us,
+    // in 256 / 320 / 384 of 8 13.2 / 17.5 / 18.0; 2^19 x 3 29.7, in 384 of 4 33.2)
+    const bool fits = !dbl || total_units <= static_cast<int64_t>(kColGroups) * e.c;
+    if (total_units < static_cast<int64_t>(kColGroups) * b.c && e.c < b.c && fits) best = id;
   }
   // 2048 points in 64 elements per thread are slower than the LDS
   // super-stage's 16 once CUs run dry (2^21 x 1: 36 against 33 us, 2048 x 1024
