@@ -240,9 +240,9 @@ int col_run_bytes(int64_t r, bool dbl, bool first) {
   return id < 0 ? 0 : kColTable[id].c * (dbl ? 16 : 8);
 }
 
-bool col_tiles_divide(int64_t r, bool dbl, int64_t tcnt) {
+bool col_tiles_divide(int64_t r, bool dbl, int64_t tcnt, int min_units) {
   for (const ColEntry &e : kColTable)
-    if (e.r == r && e.dbl == dbl && e.pref != 0 && tcnt % e.c == 0) return true;
+    if (e.r == r && e.dbl == dbl && e.c >= min_units && tcnt % e.c == 0) return true;
   return false;
 }
 

@@ -67,8 +67,8 @@ int col_kernel_id(int64_t r, bool dbl, int units, bool first);
 int col_kernel_id_for(int64_t r, bool dbl, bool first, int64_t total_units, bool rows);
 // Row-segment bytes (units x element bytes) of the default instance, 0 if none.
 int col_run_bytes(int64_t r, bool dbl, bool first);
-// Whether the tile of some instance of radix r divides tcnt units.
-bool col_tiles_divide(int64_t r, bool dbl, int64_t tcnt);
+// Whether the tile of some instance of radix r, of min_units and more, divides tcnt units.
+bool col_tiles_divide(int64_t r, bool dbl, int64_t tcnt, int min_units);
 int col_kernel_radix(int id);
 std::vector<int64_t> col_kernel_radices(bool dbl);  // the super-radices of all instances
 void col_kernel_shape(int id, int &units, int &threads, size_t &lds_bytes, int &elem_bytes);

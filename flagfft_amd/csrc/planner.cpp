@@ -187,19 +187,35 @@ int column_segment_bytes(const std::vector<int> &rad, Prec p) {
 // not divide them runs all the same, its tiles crossing sequence ends, but is
 // not priced as one: 5- and 10-smooth lengths keep their chains of 25- to
 // 1000-point passes (250000 as [125, 125, 16] would take 28 us against 32 for
-// [100, 100, 25]).
+// [100, 100, 25]).  Three things depend on the size of the whole transform:
+//   * the 4-unit FP64 tile counts up to 24 MiB (150528 x 6 as [588, 256] 31 us, [512,
+//     294] 50; but 3763200, whose 14700 256-point units only it divides, as [588, 256,
+//     25] 190, [160, 160, 147] 127);
+//   * FP64 run-time-radix passes of 512 to 1023 points, whose tiles fill a CU's LDS
+//     with one workgroup, are slower past 64 MiB (294912 x 28 as [576, 512] 265 us,
+//     [1152, 256] 186; x 7, 33 MB, 56 and 69);
+//   * FP32 ones over 2048 points between 4 and 20 MiB (150528 x 13 as [2352, 64] 66 us,
+//     [512, 294] 46; 291600 x 7 as [2160, 135] 78, [729, 400] 48; x 1 17 and 23; 602112 x
+//     13, 63 MB, as [2352, 256] 178, [1024, 588] 241).
 double pass_time(int64_t r, Prec p, bool first, const PlanOptions &o, int64_t tcnt) {
   std::vector<int> rad;
   if (o.generic_kernels) {
     // persistent-queue plans: register-resident queue instances, else the run-time-radix pass
     return (o.queue_form && col_queue_kernel_id(r, p == Prec::F64) >= 0) ? 1.0 / 4.0 : 1.0 / 1.1;
   }
-  if (o.stage_form != 2 && col_kernel_id(r, p == Prec::F64, 0) >= 0 && col_tiles_divide(r, p == Prec::F64, tcnt)) {
+  const bool dbl = p == Prec::F64;
+  const int64_t bytes = r * tcnt * elem_bytes(p) * o.nseq;
+  auto up_to = [&](int64_t mib) { return o.nseq > 0 && bytes <= mib << 20; };
+  if (o.stage_form != 2 && col_kernel_id(r, dbl, 0) >= 0 && col_tiles_divide(r, dbl, tcnt, dbl && up_to(24) ? 4 : 8)) {
     // 64-byte segments (the 4096-point instance: 8 units of 32 KiB in one
     // workgroup) run at 3.0 / 4.2, the 2048-point FP32 instance (one workgroup
     // per CU, as that one) at 3.1 / 4.1
     if (col_run_bytes(r, p == Prec::F64, first) < 128) return first ? 1.0 / 3.0 : 1.0 / 4.2;
     if (r == 2048) return first ? 1.0 / 3.1 : 1.0 / 4.1;
+    // the 512-point FP64 instance runs a little slower than its neighbours (2^18 points
+    // x 1 / 8 / 32 as [1024, 256] 15.2 / 31.1 / 98 us, as [512, 512] 16.7 / 34.3 / 113; the
+    // 2^19-point real rows that have them 16-25 % more)
+    if (r == 512 && p == Prec::F64) return first ? 1.03 / 3.8 : 1.03 / 4.6;
     return first ? 1.0 / 3.8 : 1.0 / 4.6;
   }
   if (radix_factor(r, rad)) {
@@ -208,6 +224,8 @@ double pass_time(int64_t r, Prec p, bool first, const PlanOptions &o, int64_t tc
     if (seg >= 64) return 1.0 / 3.0;
     if (seg > 0) return 1.0 / 2.2;
   }
+  if (dbl && !up_to(64) && r >= 512 && r < 1024) return 1.0 / 0.85;
+  if (!dbl && !up_to(4) && up_to(20) && r > 2048) return 1.0;
   return 1.0 / 1.1;
 }
 
@@ -611,11 +629,17 @@ PlanTree plan_tree(const PlanDesc &d, const PlanOptions &o) {
     t.rows.core.compute = d.compute;
     return t;
   }
+  auto of = [&](int64_t nseq) {
+    PlanOptions a = o;
+    a.nseq = nseq;
+    return a;
+  };
+  auto half_len = [&](int64_t n) { return d.real_fwd || d.real_inv ? n / 2 + 1 : n; };
   if (d.rank == 1) {
-    t.rows = plan_1d(d.n0, d.real_fwd, d.real_inv, d.prec, o);
+    t.rows = plan_1d(d.n0, d.real_fwd, d.real_inv, d.prec, of(d.batch));
   } else if (d.rank == 2) {
-    t.rows = plan_1d(d.n1, d.real_fwd, d.real_inv, d.prec, o);
-    t.cols = plan_1d(d.n0, false, false, d.prec, o);
+    t.rows = plan_1d(d.n1, d.real_fwd, d.real_inv, d.prec, of(d.batch * d.n0));
+    t.cols = plan_1d(d.n0, false, false, d.prec, of(d.batch * half_len(d.n1)));
     const bool half = d.real_fwd || d.real_inv;
     // one real transform whose n1 / 2 + 1 half-spectrum columns take two
     // passes only because the last tile would run alone: the DC and Nyquist
@@ -631,10 +655,10 @@ PlanTree plan_tree(const PlanDesc &d, const PlanOptions &o) {
     }
     if (!t.dc_nyq_pair) widen_columns(t.cols, d.prec, o, half ? d.n1 / 2 + 1 : d.n1, d.batch);
   } else {
-    t.rows = plan_1d(d.n2, d.real_fwd, d.real_inv, d.prec, o);
-    t.mid = plan_1d(d.n1, false, false, d.prec, o);
-    t.cols = plan_1d(d.n0, false, false, d.prec, o);
-    const int64_t n2c = (d.real_fwd || d.real_inv) ? d.n2 / 2 + 1 : d.n2;
+    const int64_t n2c = half_len(d.n2);
+    t.rows = plan_1d(d.n2, d.real_fwd, d.real_inv, d.prec, of(d.batch * d.n0 * d.n1));
+    t.mid = plan_1d(d.n1, false, false, d.prec, of(d.batch * d.n0 * n2c));
+    t.cols = plan_1d(d.n0, false, false, d.prec, of(d.batch * d.n1 * n2c));
     widen_columns(t.mid, d.prec, o, n2c, d.n0 * d.batch);
     widen_columns(t.cols, d.prec, o, d.n1 * n2c, d.batch);
   }

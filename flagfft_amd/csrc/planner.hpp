@@ -39,6 +39,7 @@ struct PlanOptions {
   int max_threads = 512;               // workgroup size limit of the launches
   bool generic_kernels = false;        // only the run-time-radix kernels (persistent-queue jobs)
   bool queue_form = false;             // with generic_kernels: register-resident passes the queue kernel runs
+  int64_t nseq = 0;                    // sequences of the planned axis (set by plan_tree; 0: many)
   bool in_place = false;               // input and output are one buffer: no sequence split over workgroups
 };
 
