@@ -221,22 +221,36 @@ flagfftResult build_plan(flagfftHandle *out, const Desc &d) {
     impl->device = dev;
     std::string tuned;
     const PlanOptions opts = plan_options(d, tuned);
-    impl->tree = plan_tree(plan_desc(d), opts);
-    const Strides *st = d.general ? &d.strides : nullptr;
-    if (d.real_fwd) {
-      impl->fwd = build_executable(impl->tree, false, opts, d.idist, d.odist, true, st);
-    } else if (d.real_inv) {
-      impl->inv = build_executable(impl->tree, true, opts, d.idist, d.odist, true, st);
-    } else {
-      impl->fwd = build_executable(impl->tree, false, opts, d.idist, d.odist, true, st);
-      impl->inv = build_executable(impl->tree, true, opts, d.idist, d.odist, true, st);
+    auto build = [&](const PlanOptions &opts) {
+      impl->fwd.reset();
+      impl->inv.reset();
+      impl->fwd_ip.reset();
+      impl->inv_ip.reset();
+      impl->tree = plan_tree(plan_desc(d), opts);
+      const Strides *st = d.general ? &d.strides : nullptr;
+      if (d.real_fwd) {
+        impl->fwd = build_executable(impl->tree, false, opts, d.idist, d.odist, true, st);
+      } else if (d.real_inv) {
+        impl->inv = build_executable(impl->tree, true, opts, d.idist, d.odist, true, st);
+      } else {
+        impl->fwd = build_executable(impl->tree, false, opts, d.idist, d.odist, true, st);
+        impl->inv = build_executable(impl->tree, true, opts, d.idist, d.odist, true, st);
+      }
+      PlanOptions ip = opts;
+      ip.in_place = true;
+      if (impl->fwd && impl->fwd->inplace_hazard)
+        impl->fwd_ip = build_executable(impl->tree, false, ip, d.idist, d.odist, true, st);
+      if (impl->inv && impl->inv->inplace_hazard)
+        impl->inv_ip = build_executable(impl->tree, true, ip, d.idist, d.odist, true, st);
+    };
+    try {
+      build(opts);
+    } catch (const std::bad_alloc &) {
+      // device memory is short: the plan with the least workspace
+      PlanOptions least = opts;
+      least.least_ws = true;
+      build(least);
     }
-    PlanOptions ip = opts;
-    ip.in_place = true;
-    if (impl->fwd && impl->fwd->inplace_hazard)
-      impl->fwd_ip = build_executable(impl->tree, false, ip, d.idist, d.odist, true, st);
-    if (impl->inv && impl->inv->inplace_hazard)
-      impl->inv_ip = build_executable(impl->tree, true, ip, d.idist, d.odist, true, st);
     std::ostringstream o;
     o << impl->tree.describe();
     if (d.general)
@@ -450,7 +464,7 @@ extern "C" flagfftResult flagfftExecZ2D(flagfftHandle plan, flagfftDoubleComplex
 // library holds one copy until the process ends.  In host code `scratch`
 // names a host-side stand-in, never the device memory: kernels get the
 // address from hipGetSymbolAddress (per device, kept in g_scratch_ptr).
-constexpr size_t kNoAllocScratchBytes = size_t(64) << 20;
+constexpr size_t kNoAllocScratchBytes = static_cast<size_t>(flagfft::kScratchBytes);
 static __device__ __align__(256) unsigned char scratch[kNoAllocScratchBytes];
 
 namespace flagfft {

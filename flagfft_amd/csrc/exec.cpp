@@ -1432,10 +1432,12 @@ void Builder::emit_bluestein(const Core &c, const SeqSet &s, int src, int dst, c
       // (two convolutions in a row per workgroup) splits in 2 below 1/2
       // (in 4 below 1/8: the combine pass reads P blocks, so P = 2 costs
       // less device time when the GPU is shared)
+      // (the split takes a workspace; with little memory only where it gains most)
       const int ncu = cu_count();
-      if (nseqs_all * 8 <= ncu || (!dbl() && !c.lds_halves && nseqs_all * 4 <= ncu))
+      const bool quarter = nseqs_all * 4 <= ncu && !opt_.least_ws;
+      if (nseqs_all * 8 <= ncu || (!dbl() && !c.lds_halves && quarter))
         split = 4;
-      else if (c.lds_halves ? nseqs_all * 2 <= ncu : nseqs_all * 4 <= ncu)
+      else if (c.lds_halves ? nseqs_all * 2 <= ncu : quarter)
         split = 2;
     }
     if (split > 0 && bluestein_split_kernel_id(M, dbl(), split) < 0) split = split == 4 ? 2 : 0;

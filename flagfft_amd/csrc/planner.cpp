@@ -300,7 +300,7 @@ double conv_time(int64_t r, Prec p, const PlanOptions &o) {
 // ones read or write the user's n <= M / 2 elements on one side).
 class ConvSplits {
  public:
-  ConvSplits(Prec p, const PlanOptions &o) {
+  ConvSplits(Prec p, const PlanOptions &o) : eb_(elem_bytes(p)), o_(o) {
     const int64_t cap = pass_max(o, p);
     const bool col_ok = o.stage_form != 2 && o.forced_units == 0;
     std::vector<int64_t> all = stage_kernel_radices();
@@ -310,8 +310,8 @@ class ConvSplits {
     for (int64_t r : all) {
       std::vector<int> rad;
       if (r > cap || !radix_factor(r, rad)) continue;
-      Radix x{r, 0.0, conv_time(r, p, o)};
       const int sid = stage_kernel_id(rad);
+      Radix x{r, 0.0, conv_time(r, p, o), sid >= 0 && stage_kernel_fast(sid)};
       if (col_ok && col_kernel_id(r, p == Prec::F64, 0) >= 0)
         x.outer = pass_time(r, p, true, o, 0) + pass_time(r, p, false, o, 0);
       else if (sid >= 0)
@@ -319,8 +319,29 @@ class ConvSplits {
       if (x.outer > 0.0 || x.conv > 0.0) rs_.push_back(x);
     }
   }
-  // The split of the cheapest M = R0 R1 in [lo, hi] (false: none).
+  // The split of the cheapest M = R0 R1 in [lo, hi] (false: none).  The chain has two
+  // workspaces of M elements per sequence, and the cheapest M is up to half longer
+  // than the shortest of fast super-radices (48197 points: 98415 = 729 x 135, 131072 =
+  // 512 x 256).  Two plans take the workspace into account:
+  //   * C2C plans that the scratch array of flagfftxExecC2CNoAlloc holds with the
+  //     shortest M take one that fits (49133 points x 38: 98415, 60 MB of 67; 131072
+  //     would need 80);
+  //   * least_ws: none longer than the shortest.
   bool best(int64_t lo, int64_t hi, std::vector<int64_t> &split) const {
+    int64_t shortest = hi;
+    for (const Radix &a : rs_)
+      for (const Radix &b : rs_)
+        if (a.fast && b.fast && a.r * b.r >= lo) shortest = std::min(shortest, a.r * b.r);
+    if (!cheapest(lo, o_.least_ws ? shortest : hi, split)) return false;
+    // (workspaces lie at 256-byte steps of the array)
+    const int64_t fit = o_.scratch_fit && o_.nseq > 0 ? kScratchBytes / 2 / 256 * 256 / eb_ / o_.nseq : 0;
+    std::vector<int64_t> s;
+    if (split[0] * split[1] > fit && shortest <= fit && cheapest(lo, fit, s)) split = s;
+    return true;
+  }
+
+ private:
+  bool cheapest(int64_t lo, int64_t hi, std::vector<int64_t> &split) const {
     double best_t = 0.0;
     for (const Radix &x1 : rs_) {
       if (x1.conv == 0.0) continue;
@@ -338,12 +359,14 @@ class ConvSplits {
     return best_t > 0.0;
   }
 
- private:
   struct Radix {
     int64_t r;
     double outer, conv;  // time as R0 / as R1, 0: no kernel
+    bool fast;           // stage_kernel_fast
   };
   std::vector<Radix> rs_;
+  int eb_;
+  PlanOptions o_;
 };
 
 bool multipass_core(int64_t n, Prec p, const PlanOptions &o, Core &c, bool by_cost = false) {
@@ -632,6 +655,7 @@ PlanTree plan_tree(const PlanDesc &d, const PlanOptions &o) {
   auto of = [&](int64_t nseq) {
     PlanOptions a = o;
     a.nseq = nseq;
+    a.scratch_fit = d.prec == Prec::F32 && !d.real_fwd && !d.real_inv;
     return a;
   };
   auto half_len = [&](int64_t n) { return d.real_fwd || d.real_inv ? n / 2 + 1 : n; };

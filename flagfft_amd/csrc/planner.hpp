@@ -17,6 +17,10 @@ namespace flagfft {
 
 enum class Prec { F32, F64 };
 
+// Workspace of flagfftxExecC2CNoAlloc (one fixed array per device): the plans it runs
+// have to stay within it.
+constexpr int64_t kScratchBytes = int64_t{64} << 20;
+
 inline int elem_bytes(Prec p) { return p == Prec::F32 ? 8 : 16; }
 
 // Tunables; defaults are the untuned heuristics, the tuned-plan DB may override.
@@ -40,6 +44,8 @@ struct PlanOptions {
   bool generic_kernels = false;        // only the run-time-radix kernels (persistent-queue jobs)
   bool queue_form = false;             // with generic_kernels: register-resident passes the queue kernel runs
   int64_t nseq = 0;                    // sequences of the planned axis (set by plan_tree; 0: many)
+  bool scratch_fit = false;            // keep convolution workspaces within kScratchBytes while a length allows it
+  bool least_ws = false;               // least workspace instead of least time (device memory is short)
   bool in_place = false;               // input and output are one buffer: no sequence split over workgroups
 };
 
@@ -112,7 +118,6 @@ int col_kernel_id(int64_t r, bool dbl, int units);
 int col_queue_kernel_id(int64_t r, bool dbl);
 int col_run_bytes(int64_t r, bool dbl, bool first);
 int col_pair_kernel_id(int64_t r, bool dbl);
-int col_kernel_id_dividing(int64_t r, bool dbl, int64_t tcnt);
 // True when every super-radix of the split has a specialised kernel (fast
 // only: one that runs near the power-of-two passes' rate).
 bool passes_specialised(const std::vector<int64_t> &passes, bool fast_only = false);

@@ -131,6 +131,10 @@ struct ServePlan {
   int64_t in_bytes = 0, out_bytes = 0;      // per transform
   std::unique_ptr<Executable> plain;        // specialised kernels, caller workspaces
   std::vector<size_t> ws_per_transform;     // plain: workspace bytes per transform
+  // the plan with the least workspace, for requests that the arena cannot hold with
+  // the plain one; made when first needed
+  std::unique_ptr<Executable> least;
+  std::vector<size_t> least_ws_per_transform;
   // The plan as persistent-queue jobs: every launch of it has a queue kind
   // (run-time-radix bodies, register-resident passes of 256 threads, real
   // split passes); step s of a batch's requests runs in the batch's s-th
@@ -144,6 +148,7 @@ struct ServePlan {
 struct Request {
   int64_t id = 0;
   ServePlan *plan = nullptr;
+  const Executable *exec = nullptr;  // plan->plain or plan->least
   int64_t batch = 0;
   const void *in = nullptr;
   size_t out_off = 0, out_size = 0;
@@ -260,20 +265,13 @@ class Server {
       if (out) *out = it->second.get();
       return FLAGFFT_SUCCESS;
     }
-    const bool real_fwd = type == FLAGFFT_R2C || type == FLAGFFT_D2Z;
-    const bool real_inv = type == FLAGFFT_C2R || type == FLAGFFT_Z2D;
-    const bool dbl = type == FLAGFFT_Z2Z || type == FLAGFFT_D2Z || type == FLAGFFT_Z2D;
-    if (!(real_fwd || real_inv || type == FLAGFFT_C2C || type == FLAGFFT_Z2Z)) return FLAGFFT_INVALID_TYPE;
+    if (!(type == FLAGFFT_R2C || type == FLAGFFT_D2Z || type == FLAGFFT_C2R || type == FLAGFFT_Z2D || type == FLAGFFT_C2C ||
+          type == FLAGFFT_Z2Z))
+      return FLAGFFT_INVALID_TYPE;
+    const PlanDesc d = desc_of(type, n);
+    const bool real_fwd = d.real_fwd, real_inv = d.real_inv, dbl = d.prec == Prec::F64;
     const int64_t h = n / 2 + 1;
     const int64_t in_len = real_inv ? h : n, out_len = real_fwd ? h : n;
-    PlanDesc d;
-    d.rank = 1;
-    d.n0 = n;
-    d.type = type;
-    d.batch = kNominalBatch;
-    d.prec = dbl ? Prec::F64 : Prec::F32;
-    d.real_fwd = real_fwd;
-    d.real_inv = real_inv;
     const bool inverse = real_inv || dir == FLAGFFT_INVERSE;
     auto sp = std::make_unique<ServePlan>();
     sp->type = type;
@@ -366,11 +364,20 @@ class Server {
     size_t need = align_up(req->out_size);
     req->queued = sp->queue &&
                   batch * (sp->in_bytes + sp->out_bytes) <= (sp->queue_fast ? queue_max_fast_ : kQueueMaxBytes);
-    for (size_t w : (req->queued ? sp->queue_ws_per_transform : sp->ws_per_transform)) {
-      req->ws_size.push_back(w * static_cast<size_t>(batch));
-      need += align_up(req->ws_size.back());
+    req->exec = sp->plain.get();
+    auto take = [&](const std::vector<size_t> &per_transform) {
+      req->ws_size.clear();
+      need = align_up(req->out_size);
+      for (size_t w : per_transform) {
+        req->ws_size.push_back(w * static_cast<size_t>(batch));
+        need += align_up(req->ws_size.back());
+      }
+      return need <= arena_.capacity();
+    };
+    if (!take(req->queued ? sp->queue_ws_per_transform : sp->ws_per_transform)) {
+      if (req->queued || !make_least(*sp, dir) || !take(sp->least_ws_per_transform)) return FLAGFFT_ALLOC_FAILED;
+      req->exec = sp->least.get();
     }
-    if (need > arena_.capacity()) return FLAGFFT_ALLOC_FAILED;
     req->arrival = Clock::now();
     {
       std::lock_guard<std::mutex> lk(mu_);
@@ -454,6 +461,42 @@ class Server {
   }
 
  private:
+  static PlanDesc desc_of(int type, int64_t n) {
+    PlanDesc d;
+    d.rank = 1;
+    d.n0 = n;
+    d.type = type;
+    d.batch = kNominalBatch;
+    d.prec = type == FLAGFFT_Z2Z || type == FLAGFFT_D2Z || type == FLAGFFT_Z2D ? Prec::F64 : Prec::F32;
+    d.real_fwd = type == FLAGFFT_R2C || type == FLAGFFT_D2Z;
+    d.real_inv = type == FLAGFFT_C2R || type == FLAGFFT_Z2D;
+    return d;
+  }
+
+  // sp.least, built at its first use (false: no plan with less workspace, or no
+  // device memory for its tables)
+  bool make_least(ServePlan &sp, int dir) {
+    std::lock_guard<std::mutex> lk(plans_mu_);
+    if (!sp.least) {
+      const PlanDesc d = desc_of(sp.type, sp.n);
+      const int64_t h = sp.n / 2 + 1;
+      PlanOptions o;
+      o.least_ws = true;
+      try {
+        auto ex = build_executable(plan_tree(d, o), d.real_inv || dir == FLAGFFT_INVERSE, o, d.real_inv ? h : sp.n,
+                                   d.real_fwd ? h : sp.n, false);
+        std::vector<size_t> per;
+        for (size_t b : ex->ws_bytes) per.push_back(b / static_cast<size_t>(kNominalBatch));
+        table_bytes_ += tables_of(*ex);
+        sp.least_ws_per_transform = std::move(per);
+        sp.least = std::move(ex);
+      } catch (const std::exception &) {
+        return false;
+      }
+    }
+    return true;
+  }
+
   static size_t tables_of(const Executable &ex) {
     size_t b = 0;
     for (const auto &kv : ex.tables) b += kv.second->bytes;
@@ -754,7 +797,7 @@ class Server {
     for (Request *r : direct) {
       std::vector<void *> ws;
       for (size_t o : r->ws_off) ws.push_back(base + o);
-      e = r->plan->plain->run_batch(r->in, base + r->out_off, ws.data(), r->batch, slot.stream);
+      e = r->exec->run_batch(r->in, base + r->out_off, ws.data(), r->batch, slot.stream);
       if (e != hipSuccess) return e;
       Group g;
       g.ev = take_event_unlocked();
