@@ -211,7 +211,7 @@ int col_kernel_id(int64_t r, bool dbl, int units, bool first) {
 
 int col_kernel_id(int64_t r, bool dbl, int units) { return col_kernel_id(r, dbl, units, false); }
 
-int col_kernel_id_for(int64_t r, bool dbl, bool first, int64_t total_units, bool rows) {
+int col_kernel_id_for(int64_t r, bool dbl, bool first, int64_t total_units, bool rows, bool complex_ends) {
   const int n = static_cast<int>(sizeof(kColTable) / sizeof(kColTable[0]));
   // first 256-point passes of long 1D batches read 512-byte runs as the later
   // ones do (65536 x 128 48.0 -> 45.3 us, x 256 95.5 -> 89.4, x 64 the same; 256^3
@@ -230,8 +230,10 @@ int col_kernel_id_for(int64_t r, bool dbl, bool first, int64_t total_units, bool
   }
   // 2048 points in 64 elements per thread are slower than the LDS
   // super-stage's 16 once CUs run dry (2^21 x 1: 36 against 33 us, 2048 x 1024
-  // columns: 20 against 18); 4096 points are not (2^22 x 1: 40 against 44)
-  if (r == 2048 && total_units < static_cast<int64_t>(kColGroups) * kColTable[best].c) return -1;
+  // columns: 20 against 18); 4096 points are not (2^22 x 1: 40 against 44).  Real and
+  // Hermitian ends of a convolution have no super-stage, only the run-time-radix pass
+  // of a fourth launch (R2C 1000003 x 1: 77 us, here 54; 160001 x 8: 147 and 53)
+  if (complex_ends && r == 2048 && total_units < static_cast<int64_t>(kColGroups) * kColTable[best].c) return -1;
   return best;
 }
 

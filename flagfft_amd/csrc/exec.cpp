@@ -888,6 +888,8 @@ bool Builder::try_stage(const PassArgs &a, const std::vector<int> &radices, int 
   const int sid = opt_.generic_kernels        ? -1
                   : opt_.forced_units != 0 ? stage_kernel_id(radices, dbl(), opt_.forced_units)
                                            : stage_kernel_id_for(radices, dbl(), a.units);
+  // (the LDS super-stage reads and writes complex sequences only)
+  const bool complex_ends = (a.src_mode & 3) == kSrcComplex && (a.dst_mode & 3) == kDstComplex;
   // register-resident two-stage pass (plain complex passes, and Bluestein
   // chain ends: chirp source, pointwise and chirp sinks)
   const bool col_allowed = mode == 0 && opt_.stage_form != 2 && (!opt_.generic_kernels || opt_.queue_form) &&
@@ -899,7 +901,7 @@ bool Builder::try_stage(const PassArgs &a, const std::vector<int> &radices, int 
             : opt_.queue_form ? col_queue_kernel_id(a.R, dbl())
             : opt_.forced_units != 0
                 ? col_kernel_id(a.R, dbl(), opt_.forced_units, a.p == 1)
-                : col_kernel_id_for(a.R, dbl(), a.p == 1, a.units, !s.col_fast);
+                : col_kernel_id_for(a.R, dbl(), a.p == 1, a.units, !s.col_fast, complex_ends);
   // DC / Nyquist pair: one transform's single column pass over the n1 / 2
   // columns of the half spectrum (row pitch n1 / 2 + 1) but its Nyquist
   // column, which goes with column 0; the other side is a workspace of n1 / 2
@@ -913,8 +915,6 @@ bool Builder::try_stage(const PassArgs &a, const std::vector<int> &radices, int 
     cid = col_pair_kernel_id(a.R, dbl());
     if (cid < 0) throw std::logic_error("DC/Nyquist pair: no paired column instance");
   }
-  // (the LDS super-stage reads and writes complex sequences only)
-  const bool complex_ends = (a.src_mode & 3) == kSrcComplex && (a.dst_mode & 3) == kDstComplex;
   if ((sid < 0 && cid < 0) || (cid < 0 && !complex_ends)) return false;
   // contiguous sequences, or the columns of contiguous rows of ncol elements
   const bool rows = !s.col_fast && s.ncol == 1 && a.gi.es == 1 && a.go.es == 1;
@@ -1390,12 +1390,13 @@ void Builder::emit_bluestein_split(const Core &c, const SeqSet &s, int src, int 
 }
 
 // Whether the outer launches of a two-pass Bluestein convolution of length M
-// with super-radix r0 run on register-resident instances for these sequences.
+// with super-radix r0 run on register-resident instances for these sequences, whose
+// real or Hermitian elements no other kernel of the three launches reads or writes.
 bool Builder::conv_ends_in_registers(int64_t r0, int64_t M, const SeqSet &s) {
   if (opt_.stage_form == 2 || opt_.forced_units != 0) return false;
   const int64_t tcnt = M / r0;
   for (bool first : {true, false}) {
-    const int id = col_kernel_id_for(r0, dbl(), first, s.nbatch * tcnt, true);
+    const int id = col_kernel_id_for(r0, dbl(), first, s.nbatch * tcnt, true, false);
     int units = 0, threads = 0, ebytes = 0;
     size_t lds = 0;
     if (id < 0) return false;

@@ -63,8 +63,8 @@ int col_kernel_id(int64_t r, bool dbl, int units, bool first);
 // The default instance for a launch of total_units units (rows: of contiguous
 // sequences, not columns): a narrower tile when
 // the default one would leave CUs without a workgroup, -1 where the LDS
-// super-stage is faster for so few.
-int col_kernel_id_for(int64_t r, bool dbl, bool first, int64_t total_units, bool rows);
+// super-stage, which reads and writes complex sequences only, is faster for so few.
+int col_kernel_id_for(int64_t r, bool dbl, bool first, int64_t total_units, bool rows, bool complex_ends);
 // Row-segment bytes (units x element bytes) of the default instance, 0 if none.
 int col_run_bytes(int64_t r, bool dbl, bool first);
 // Whether the tile of some instance of radix r, of min_units and more, divides tcnt units.
