@@ -62,8 +62,8 @@ __device__ __forceinline__ void stt_nt(GlbC<T> *base, uint32_t idx, V2<T> v) {
 // a relative L2 error of 2.75e-7 that way and 2.03e-7 with the three values,
 // for 1 % of their time.  Passes of 16 elements per thread keep the one load
 // (with three, twice the loads of their data: second pass of 65536 x 256 44.5 ->
-// 46.7 us) unless they stand in for the run-time-radix pass with its table of
-// all powers, in Bluestein chains of real sequences.
+// 46.7 us) unless they are an end of a Bluestein chain, where they stand in for the
+// run-time-radix pass with its table of all powers.
 template <int N, bool EXACT, typename T, typename Get>
 __device__ __forceinline__ void powers(Get get, V2<T> *p) {
   p[0] = V2<T>{1, 0};

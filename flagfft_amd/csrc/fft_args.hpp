@@ -278,7 +278,7 @@ struct RealPassArgs {
 // chain whose earlier passes ran in an earlier queue launch), with the
 // arguments of the equivalent standalone launch (run-time-radix kinds: FP32
 // with 16 elements per thread, FP64 with 8; register-resident passes: the
-// queue instance `variant` of 256 threads).
+// queue instance of 256 threads that `variant` names).
 enum QueueKind : int32_t {
   kQueuePass = 0,
   kQueueRader = 1,
@@ -294,7 +294,7 @@ struct QueueJob {
   int32_t dbl;
   int32_t first;    // index of the job's first tile in the launch
   int32_t nblocks;  // tiles
-  int32_t variant;  // kQueueCol: queue instance of the register-resident pass
+  int32_t variant;  // kQueueCol: 2 x queue instance of the register-resident pass (+ 1: Bluestein ends)
   int32_t pad_;
   union {
     PassArgs pa;      // kQueuePass

@@ -734,12 +734,14 @@ __global__ __launch_bounds__(kQueueThreads) void k_queue(const QueueArgs q) {
 }
 
 // ---------------------------------------------------------------------------
-// Persistent kernels of the register-resident passes: one per instance (the
-// queue variants of colpass.hip's catalogue), each draining the jobs of that
-// instance with k_queue's tile loop, so that every instance keeps its own
-// register count (a kernel holding several would need the registers of all).
+// Persistent kernels of the register-resident passes: two per instance (the
+// queue variants of colpass.hip's catalogue), for plain passes and for Bluestein
+// chain ends as the standalone kernels are, each draining the jobs of that
+// kind with k_queue's tile loop, so that every one keeps its own register
+// count: a kernel of both forms spills 16 (1024 points), 44 (512) and 33 (256) VGPRs,
+// the Bluestein form 10, 0 and 16, the plain one 0, 0 and 1.
 // ---------------------------------------------------------------------------
-template <typename T, int C, int RA, int RB, int NCH, int WPE>
+template <typename T, int C, int RA, int RB, int NCH, int WPE, int MODE>
 __global__ __launch_bounds__(kQueueThreads) __attribute__((amdgpu_waves_per_eu(WPE))) void k_queue_col(const QueueArgs q) {
   __shared__ int item_s;
   for (;;) {
@@ -769,7 +771,8 @@ __global__ __launch_bounds__(kQueueThreads) __attribute__((amdgpu_waves_per_eu(W
 #pragma unroll
     for (int w = 0; w < NW; ++w) u.w[w] = __builtin_amdgcn_readlane(mine, w);
     const int first = __builtin_amdgcn_readfirstlane(q.jobs[lo].first);
-    col_body<T, C, RA, RB, NCH, kColBluestein>(u.a, item - first);
+    if constexpr (MODE == kColPlain) u.a.stream = 0;  // small requests: no cache hints, and no registers for them
+    col_body<T, C, RA, RB, NCH, MODE>(u.a, item - first);
   }
 }
 
@@ -998,22 +1001,27 @@ const void *r2c_even_kernel(bool dbl, int ept) { FLAGFFT_KERNEL_EPT(k_r2c_even);
 const void *c2r_even_kernel(bool dbl, int ept) { FLAGFFT_KERNEL_EPT(k_c2r_even); }
 
 const void *queue_kernel() { return reinterpret_cast<const void *>(dev::k_queue); }
-// Indexed by QueueJob::variant (colpass.hip's queue variants); null where unused.
+// Indexed by QueueJob::variant (colpass.hip's queue variants, each plain and with
+// Bluestein chain ends); null where unused.
+#define FLAGFFT_QUEUE_COL(...)                                                          \
+  reinterpret_cast<const void *>(dev::k_queue_col<__VA_ARGS__, dev::kColPlain>), \
+      reinterpret_cast<const void *>(dev::k_queue_col<__VA_ARGS__, dev::kColBluestein>)
 const void *queue_col_kernel(int variant) {
   static const void *const k[] = {
-      reinterpret_cast<const void *>(dev::k_queue_col<float, 8, 32, 32, 2, 4>),
-      reinterpret_cast<const void *>(dev::k_queue_col<float, 16, 32, 16, 1, 2>),
-      reinterpret_cast<const void *>(dev::k_queue_col<float, 16, 16, 16, 1, 4>),
-      reinterpret_cast<const void *>(dev::k_queue_col<float, 32, 16, 8, 1, 3>),
-      reinterpret_cast<const void *>(dev::k_queue_col<float, 32, 8, 8, 1, 4>),
-      reinterpret_cast<const void *>(dev::k_queue_col<float, 64, 8, 4, 1, 4>),
-      reinterpret_cast<const void *>(dev::k_queue_col<float, 64, 4, 4, 1, 4>),
-      reinterpret_cast<const void *>(dev::k_queue_col<double, 16, 16, 16, 1, 2>),
-      nullptr,
-      reinterpret_cast<const void *>(dev::k_queue_col<double, 32, 8, 8, 1, 4>),
+      FLAGFFT_QUEUE_COL(float, 8, 32, 32, 2, 4),
+      FLAGFFT_QUEUE_COL(float, 16, 32, 16, 1, 2),
+      FLAGFFT_QUEUE_COL(float, 16, 16, 16, 1, 4),
+      FLAGFFT_QUEUE_COL(float, 32, 16, 8, 1, 3),
+      FLAGFFT_QUEUE_COL(float, 32, 8, 8, 1, 4),
+      FLAGFFT_QUEUE_COL(float, 64, 8, 4, 1, 4),
+      FLAGFFT_QUEUE_COL(float, 64, 4, 4, 1, 4),
+      FLAGFFT_QUEUE_COL(double, 16, 16, 16, 1, 2),
+      nullptr, nullptr,
+      FLAGFFT_QUEUE_COL(double, 32, 8, 8, 1, 4),
   };
   return variant >= 0 && variant < static_cast<int>(sizeof(k) / sizeof(k[0])) ? k[variant] : nullptr;
 }
+#undef FLAGFFT_QUEUE_COL
 
 const void *real_post_kernel(bool dbl) {
   return dbl ? reinterpret_cast<const void *>(dev::k_real_post<double>)

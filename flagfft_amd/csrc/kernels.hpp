@@ -79,7 +79,7 @@ const void *col_kernel(int id, bool bluestein);  // bluestein: with the modes of
 const void *col_pair_kernel(int id);
 int col_pair_kernel_id(int64_t r, bool dbl);
 // The instance of 256 threads the persistent queue kernel also runs (-1 if
-// none for r), and its queue variant (QueueJob::variant; -1 for others).
+// none for r), and its queue variant (half of QueueJob::variant; -1 for others).
 int col_queue_kernel_id(int64_t r, bool dbl);
 int col_queue_variant(int id);
 // The instance whose convolution launch (k_col_conv) a Bluestein chain of
@@ -100,7 +100,7 @@ std::string col_kernel_targs(int id, int mode);  // mode: ColMode
 // QueueArgs argument).
 const void *queue_kernel();
 // Persistent kernel of the register-resident pass jobs (kQueueCol) of one
-// queue variant (QueueJob::variant), null if none.
+// QueueJob::variant, null if none.
 const void *queue_col_kernel(int variant);
 
 // Bluestein kernels with the convolution in LDS (FP32): id for the

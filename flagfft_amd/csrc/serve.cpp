@@ -47,9 +47,10 @@ constexpr int64_t kQueueMaxBytes = int64_t{32} << 20;   // larger requests with 
 constexpr int64_t kQueueMaxBytesFast = int64_t{64} << 20;
 constexpr int kMaxQueueSteps = 6;                       // queue launches per batch (passes of the longest plan)
 // queue launches per batch: per step, the run-time-radix kernel and one per
-// register-resident variant present (at most 10)
-constexpr int kMaxQueueLaunches = kMaxQueueSteps * 11;
-constexpr size_t kStagingBytes = 256 * kMaxQueueLaunches + sizeof(QueueJob) * kMaxJobs * kMaxQueueSteps;
+// register-resident variant present (at most 20)
+constexpr int kMaxQueueLaunches = kMaxQueueSteps * 21;
+// (per launch a counter's kAlign bytes, and its jobs rounded up to kAlign)
+constexpr size_t kStagingBytes = 2 * kAlign * kMaxQueueLaunches + sizeof(QueueJob) * kMaxJobs * kMaxQueueSteps;
 constexpr int64_t kNominalBatch = 512;             // batch the cached plans are shaped for
 constexpr double kLargeRequestBytes = 64.0 * (1 << 20);  // direct requests above this stay in arrival order
 // ... on lane 0 unless this many requests wait (pending admission or
@@ -184,8 +185,8 @@ bool queue_kind_of(const Step &s, int &kind, int &variant) {
   switch (s.kind) {
     case Step::Col:
       kind = kQueueCol;
-      variant = col_queue_variant(s.leaf_id);
-      return variant >= 0 && s.shape.block.x == static_cast<unsigned>(kQueueThreads) &&
+      variant = 2 * col_queue_variant(s.leaf_id) + (s.leaf_mode == 3 ? 1 : 0);
+      return variant >= 0 && (s.leaf_mode == 0 || s.leaf_mode == 3) && s.shape.block.x == static_cast<unsigned>(kQueueThreads) &&
              s.shape.lds_bytes <= 80 * 1024;
     case Step::RealPost:
     case Step::RealPre:
