@@ -198,6 +198,12 @@ struct StageEntry {
   {2, {R0, R1, 0}, C32, E32, C64, E64, FLAGFFT_STAGE_FNS(C32, E32, C64, E64, R0, R1), true}
 #define FLAGFFT_STAGE3(C32, E32, C64, E64, R0, R1, R2) \
   {3, {R0, R1, R2}, C32, E32, C64, E64, FLAGFFT_STAGE_FNS(C32, E32, C64, E64, R0, R1, R2), true}
+// (FP32 alone: c64 = 0)
+#define FLAGFFT_STAGE3_F32(C32, E32, R0, R1, R2)                                                     \
+  {3, {R0, R1, R2}, C32, E32, 0, 0,                                                                  \
+   {{(const void *)dev::k_stage<float, E32, C32, dev::kStagePass, R0, R1, R2>,                       \
+     (const void *)dev::k_stage<float, E32, C32, dev::kStageConvolution, R0, R1, R2>},               \
+    {nullptr, nullptr}}, true}
 #define FLAGFFT_STAGE2_SLOW(C32, E32, C64, E64, R0, R1) \
   {2, {R0, R1, 0}, C32, E32, C64, E64, FLAGFFT_STAGE_FNS(C32, E32, C64, E64, R0, R1), false}
 #define FLAGFFT_STAGE3_SLOW(C32, E32, C64, E64, R0, R1, R2) \
@@ -236,7 +242,7 @@ const StageEntry kStageTable[] = {
     // largest radix per thread (a launch of 32-63 workgroups is latency: 1000 x 1000
     // columns 30.4 -> 10.4 us, 10^6 x 1 57 -> 18, 729 x 729 columns 20.6 -> 8.8,
     // 100 x 100 columns 14.3 -> 6.4)
-    FLAGFFT_STAGE3(4, 9, 4, 9, 9, 9, 9),           // 729
+    FLAGFFT_STAGE3_F32(4, 9, 9, 9, 9),             // 729 (FP64: its default tile is this narrow)
     FLAGFFT_STAGE2_SLOW(8, 10, 8, 10, 10, 10),     // 100
     FLAGFFT_STAGE3_SLOW(8, 5, 8, 5, 5, 5, 5),      // 125
     FLAGFFT_STAGE3_SLOW(4, 10, 4, 10, 10, 10, 10), // 1000
@@ -267,7 +273,7 @@ int stage_kernel_id_for(const std::vector<int> &radices, bool dbl, int64_t total
     const StageEntry &e = kStageTable[i], &b = kStageTable[best];
     if (e.nrad != b.nrad || !std::equal(e.rad, e.rad + 3, b.rad)) continue;
     const int c = dbl ? e.c64 : e.c32, bc = dbl ? b.c64 : b.c32;
-    if (c < bc && total_units < int64_t{256} * bc) best = i;
+    if (c > 0 && c < bc && total_units < int64_t{256} * bc) best = i;
   }
   return best;
 }
