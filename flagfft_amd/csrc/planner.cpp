@@ -612,14 +612,15 @@ void widen_columns(Plan1D &cols, Prec prec, const PlanOptions &o, int64_t ncol, 
   // 95 us for two 64-point passes), when its workgroups (one per CU) fill the
   // 256 CUs in whole rounds (2049 half-spectrum columns are 257 tiles: the
   // last one would run alone, 228 against 173 us for the 4096^2 R2C->C2R
-  // step) and tile whole transforms
+  // step).  Tiles may cross the ends of transforms (16 x 4096 x 500 R2C, whose 251
+  // columns 8 units do not divide: 310 us as two passes, 265 so)
   const int run = o.stage_form != 2 ? col_run_bytes(cols.n, prec == Prec::F64, false) : 0;
   if (run >= 64) {
     constexpr int64_t kCus = 256;
     const int64_t c = run / elem_bytes(prec);
     const int64_t tiles = (ncol * nseq + c - 1) / c;
     const int64_t rounds = (tiles + kCus - 1) / kCus;
-    if ((nseq == 1 || ncol % c == 0) && 4 * tiles >= 3 * rounds * kCus) return;
+    if (4 * tiles >= 3 * rounds * kCus) return;
   }
   // (no LDS super-stage instance for the whole column either: the
   // run-time-radix pass would read it one element per column)
