@@ -43,7 +43,7 @@ def test_results_complex(gpu, n0, n2):
         sync(gpu)
     y = host(yd)
     assert (y[x.size:] == 7.0).all()
-    check_accuracy(y[:x.size].reshape(x.shape), np.fft.fftn(x.astype(np.complex128)), ff.Type.C2C, x.size, row_len=n2)
+    check_accuracy(y[:x.size].reshape(x.shape), np.fft.fftn(x.astype(np.complex128)), ff.Type.C2C, x.size, row_len=x.size)
 
 
 @pytest.mark.gpu
@@ -59,4 +59,5 @@ def test_results_real(gpu):
         sync(gpu)
     y = host(yd)
     assert (y[n0 * N1 * h:] == 7.0).all()
-    check_accuracy(y[:n0 * N1 * h].reshape(n0, N1, h), np.fft.rfftn(x.astype(np.float64)), ff.Type.R2C, x.size, row_len=h)
+    check_accuracy(y[:n0 * N1 * h].reshape(n0, N1, h), np.fft.rfftn(x.astype(np.float64)), ff.Type.R2C, x.size,
+                   row_len=n0 * N1 * h)
