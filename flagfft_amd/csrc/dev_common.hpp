@@ -162,11 +162,12 @@ __device__ __forceinline__ void dst_elem(void *out, int64_t base, int64_t es, in
 // serialising one per loop iteration.
 // With FULL, batches end in loads of the last element again instead of masked loads
 // (a load under a mask waits for the one before it: the generic pass gains 5-15 %,
-// the real and prime kernels lose 10 % to the registers).  Totals of at most U / 2
-// elements per thread stop there: the repeats' address arithmetic would cost more
-// than the data (axes of 1 / 3 / 4 elements, 1024 x 2048 of them, 81 -> 71, 146 -> 132,
-// 167 -> 148 us, masked 69, 137, 168; a second stop at two elements costs longer ones 2 %).
-template <typename T, int U, bool FULL = false, typename Load, typename Commit>
+// the real and prime kernels lose 10 % to the registers).  With STOP, totals of at
+// most U / 2 elements per thread stop there: the repeats' address arithmetic would
+// cost more than the data (axes of 1 / 3 / 4 elements, 1024 x 2048 of them, 81 -> 71,
+// 146 -> 132, 167 -> 148 us, masked 69, 137, 168; a second stop at two elements costs
+// longer ones 2 %, a stop where loads are twiddled 5 %: FP64 35-point passes 44 -> 46).
+template <typename T, int U, bool FULL = false, bool STOP = false, typename Load, typename Commit>
 __device__ __forceinline__ void batched(int total, int tid, int nthr, Load load, Commit commit) {
   for (int f0 = tid; f0 < total; f0 += U * nthr) {
     V2<T> v[U];
@@ -174,7 +175,7 @@ __device__ __forceinline__ void batched(int total, int tid, int nthr, Load load,
     for (int uu = 0; uu < U; ++uu) {
       const int f = f0 + uu * nthr;
       if constexpr (FULL) {
-        if (uu == U / 2 && total <= uu * nthr) break;
+        if (STOP && uu == U / 2 && total <= uu * nthr) break;
         v[uu] = load(min(f, total - 1));
       } else if (f < total) {
         v[uu] = load(f);

@@ -321,7 +321,7 @@ __device__ __forceinline__ void pass_body(const PassArgs &a, int blk) {
   };
   // (slots past the last unit read it again; their results are not stored)
   auto fill = [&](auto source, auto twiddled) __attribute__((always_inline)) {
-    batched<T, kBatch, true>(
+    batched<T, kBatch, true, !decltype(twiddled)::value>(
         CR, tid, nthr,
         [&](int f) __attribute__((always_inline)) {
           int s, e;
