@@ -37,9 +37,10 @@ constexpr int64_t kStreamHalfRowBytes = int64_t{2} << 20, kStreamHalfRowShort = 
 // Outputs of a split-spectrum pass of its own (k_real_post) from this size on:
 // smaller ones are faster left in the caches (R2C then C2R of 1002 points x 2092, 8
 // MiB, 84.5 us without and 85.6 with the hint, 752 x 8366, 24 MiB, 233.8 and 235.1),
-// larger ones written around them (1002 x 12557, 48 MiB, R2C 251 -> 222, there and
+// larger ones written around them (D2Z 875000 x 5, 33 MiB, 103 -> 98, there and back
+// 204 -> 202; 1002 x 12557, 48 MiB, R2C 251 -> 222, there and
 // back the same; 200000 x 131 163 -> 146, 328 -> 316; 2^25 183 -> 174, 390 -> 375).
-constexpr int64_t kStreamPostBytes = int64_t{40} << 20;
+constexpr int64_t kStreamPostBytes = int64_t{32} << 20;
 }  // namespace
 
 void hip_check(hipError_t e, const char *what) {
@@ -280,7 +281,9 @@ void Step::set_stream_hints() {
       // a streamed line does not wait for (64-byte segments: second pass of
       // 2^24 62 -> 86 us; 128 bytes: 2^20 x 16 107 -> 99 us, 512: 65536 x 256
       // 93.5 -> 87.5).  Columns of 2D / 3D arrays keep plain stores: a
-      // following transform reads them sooner (256^3 there and back 249 -> 261)
+      // following transform reads them sooner (256^3 there and back 249 -> 261).
+      // 1D chains pay that too: outputs of 64 MiB 0.72-0.90 of the plain time one
+      // way, 1.03-1.10 there and back; from 256 MiB on 0.75-0.9 both, to 24 MiB even
       int units = 0, threads = 0, eb = 0;
       size_t lds = 0;
       col_kernel_shape(leaf_id, units, threads, lds, eb);

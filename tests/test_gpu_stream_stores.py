@@ -24,7 +24,7 @@ def test_rows(gpu, kind, n, batch, parts, whole, part):
     _compare(gpu, kind, n, batch, parts, whole, part)
 
 
-# the split-spectrum pass of its own, lines at 40 MiB
+# the split-spectrum pass of its own, lines at 32 MiB
 POST = [("r2c", 752, 20000, 2, True, False), ("d2z", 1502, 5000, 2, True, False), ("r2c", 200000, 60, 2, True, False)]
 
 

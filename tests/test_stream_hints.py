@@ -64,9 +64,9 @@ def test_row_stores(standin):
         assert len(steps) == 1 and steps[0][2] == want, (t, n, b, steps)
 
 
-# the split-spectrum pass of its own: from 40 MiB on
-POST = [("R2C", 752, 419, False), ("R2C", 752, 13900, False), ("R2C", 752, 13920, True), ("D2Z", 1502, 3400, False),
-        ("D2Z", 1502, 3500, True), ("R2C", 1 << 25, 1, True)]
+# the split-spectrum pass of its own: from 32 MiB on
+POST = [("R2C", 752, 419, False), ("R2C", 752, 11100, False), ("R2C", 752, 11140, True), ("D2Z", 1502, 2780, False),
+        ("D2Z", 1502, 2800, True), ("R2C", 1 << 25, 1, True)]
 
 
 def test_split_spectrum_pass(standin):
