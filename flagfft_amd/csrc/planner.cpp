@@ -194,9 +194,10 @@ int column_segment_bytes(const std::vector<int> &rad, Prec p) {
 //   * FP64 run-time-radix passes of 512 to 1023 points, whose tiles fill a CU's LDS
 //     with one workgroup, are slower past 64 MiB (294912 x 28 as [576, 512] 265 us,
 //     [1152, 256] 186; x 7, 33 MB, 56 and 69);
-//   * FP32 ones over 2048 points between 4 and 20 MiB (150528 x 13 as [2352, 64] 66 us,
-//     [512, 294] 46; 291600 x 7 as [2160, 135] 78, [729, 400] 48; x 1 17 and 23; 602112 x
-//     13, 63 MB, as [2352, 256] 178, [1024, 588] 241).
+//   * FP32 ones over 2048 points, a workgroup per unit, once a CU has more than one, to
+//     20 MiB (150528 x 4 / 5 / 13 as [2352, 64], 256 / 320 / 832 units, 22 / 36 / 66 us, as
+//     [512, 294] 28 / 28 / 46; 291600 x 2 as [2160, 135], 270 units, 41, [2916, 100], 200,
+//     25.5, [729, 400] 25.3; 602112 x 13, 63 MB, as [2352, 256] 178, [1024, 588] 241).
 double pass_time(int64_t r, Prec p, bool first, const PlanOptions &o, int64_t tcnt) {
   std::vector<int> rad;
   if (o.generic_kernels) {
@@ -225,7 +226,7 @@ double pass_time(int64_t r, Prec p, bool first, const PlanOptions &o, int64_t tc
     if (seg > 0) return 1.0 / 2.2;
   }
   if (dbl && !up_to(64) && r >= 512 && r < 1024) return 1.0 / 0.85;
-  if (!dbl && !up_to(4) && up_to(20) && r > 2048) return 1.0;
+  if (!dbl && tcnt * o.nseq > 256 && up_to(20) && r > 2048) return 1.0;
   return 1.0 / 1.1;
 }
 

@@ -17,8 +17,9 @@ SPLITS = [("Z2Z", 262144, 1, [1024, 256]), ("Z2Z", 262144, 64, [1024, 256]), ("D
           ("Z2Z", 150528, 6, [588, 256]), ("Z2Z", 150528, 13, [512, 294]), ("Z2Z", 3763200, 1, [160, 160, 147]),
           # run-time-radix passes of 512 to 1023 points past 64 MiB
           ("Z2Z", 294912, 7, [576, 512]), ("Z2Z", 294912, 28, [1152, 256]),
-          # FP32 ones over 2048 points between 4 and 20 MiB
-          ("C2C", 150528, 1, [2352, 64]), ("C2C", 150528, 13, [512, 294]), ("C2C", 291600, 7, [729, 400]),
+          # FP32 ones over 2048 points with more than 256 units, to 20 MiB
+          ("C2C", 150528, 1, [2352, 64]), ("C2C", 150528, 4, [2352, 64]), ("C2C", 150528, 5, [512, 294]),
+          ("C2C", 602112, 1, [2352, 256]), ("C2C", 291600, 1, [2160, 135]), ("C2C", 291600, 2, [2916, 100]), ("C2C", 150528, 13, [512, 294]), ("C2C", 291600, 7, [729, 400]),
           ("C2C", 602112, 13, [2352, 256])]
 
 
