@@ -170,7 +170,7 @@ __device__ __forceinline__ void col_load(const StageArgs &a, int blk, V2<T> (&x)
   // drift apart, so that loads, arithmetic and stores of a CU's workgroups
   // overlap: 65536 x 16 12.9 us straight, 12.7 masked, R2C of 2^15 x 8 10.8 and 10.4, 155
   // chains, images and volumes 1.5 % in the mean.  Not the tile whose unit 0 is a pair: its lanes left above.)
-  const bool straight = RA >= 64 || a.p == a.ncol;
+  const bool straight = RA >= 64 || MODE == kColRealPre || (MODE != kColRealPost && a.p == a.ncol);
   if (straight && !chirp_in && un.whole && !(MODE == kColPair && a.dc_nyq_pair == 2 && blk == 0)) {
     auto load_tile = [&](auto ld) __attribute__((always_inline)) {
 #pragma unroll
